@@ -30,6 +30,18 @@ from . import simplify
 
 BLOCK = 256
 LDS_BYTES = 32768          # privatised tallies per block (MI355X: 160 KB LDS per CU)
+LDS_F64 = 8192             # of those, float32 sums held as float64 in LDS take up to this many bytes (8 per bin):
+                           # ds_add_f64 runs ~8x faster than ds_add_f32 on gfx950 (a wave64 add occupies a CU's LDS
+                           # for ~6 cycles against 194 -- 2,048 workgroups x 256 x 512 adds onto 64 random bins:
+                           # 0.167 ms, 0.13 of it the address arithmetic, against 1.335 -- whatever the bins and
+                           # conflicts), and a float32 value or a sum of them is never a float64 subnormal, so the
+                           # compare-and-swap path of tm_ladd_f32 goes too.  Larger tallies keep float32: at 8 bytes a
+                           # 4,096-bin map takes a workgroup per CU from the loop, and there the adds are not the bound
+LDS_COPIES = 256           # a float64 or count bin of a tally of S bins has up to 16 copies in LDS, S x copies at most
+                           # this (8-byte words); a lane adds to copy lane % copies and the flush sums them.  Lanes of
+                           # a wave that add to one address take turns: ds_add_f64 cycles per wave64 add and CU (the
+                           # probe above, ~18 of them address arithmetic) 392 onto one bin, 111 onto 2, 45 onto 8, 31
+                           # onto 16, 24 onto 64; with 16 copies 18-19 onto 1, 8 or 16 bins, with 4 copies 21 onto 64
 REG_BINS = 2               # privatised tallies of at most this many bins accumulate in each lane's registers
 XW = 9                     # int64 words per exact bin (tm_device.h TM_XW: weights 2^(32 j))
 CHUNK = 64
@@ -418,6 +430,34 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     # per bin, merged into the workgroup's copy once when the lane exits: no LDS atomic per emit.  (An exact tally
     # would take 2 x XW registers per bin in every lane -- measured slower on C5's reverse launch -- so it stays in
     # LDS.)
+    # float32 sums accumulated as float64 in LDS (LDS_F64), rounded once per workgroup by the flush
+    d64, left = set(), LDS_F64
+    for k in priv:
+        s = prog.tallies[k]
+        if s.dtype == C.F32 and not s.exact and not s.fixed and 8 * s.S <= left:
+            left -= 8 * s.S
+            d64.add(k)
+
+    def copies(S, words):
+        """LDS copies per bin of an 8-byte accumulator of S bins, while all of them fit `words`."""
+        R = 16
+        while R > 1 and (S * R > LDS_COPIES or S * R > words):
+            R //= 2
+        return R
+    ncopy, words = {}, LDS_F64 // 8
+    for k in priv:
+        s = prog.tallies[k]
+        if k in d64 or (s.dtype == C.F64 and not s.fixed):
+            ncopy[k] = copies(s.S, words)
+            words -= s.S * ncopy[k] if ncopy[k] > 1 else 0
+
+    def copy_of(ei, R):
+        """the index of bin ei's copy for this lane."""
+        return ei if R == 1 else f"{ei} * {R} + (threadIdx.x & {R - 1}u)"
+
+    def sum_copies(nm, R):
+        """the flush's total of bin i's copies (a C expression)."""
+        return f"{nm}[i]" if R == 1 else "(" + " + ".join(f"{nm}[i * {R} + {q}]" for q in range(R)) + ")"
     rpriv = [k for k in priv if prog.tallies[k].S <= REG_BINS and not prog.tallies[k].fixed
              and not prog.tallies[k].exact and prog.tallies[k].dtype in (C.F32, C.I32, C.U32)]
     em = Emitter()
@@ -466,7 +506,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             key = (k, int(c.view(np.uint32)))
             if key not in counts:
                 counts[key] = (f"tm_cn{k}_{len(counts)}", c)
-            em_.line(f"atomicAdd(&{counts[key][0]}[{ei}], 1ull);")
+            em_.line(f"atomicAdd(&{counts[key][0]}[{copy_of(ei, copies(s.S, LDS_F64))}], 1ull);")
             em_.close()
             return t
         if s.exact:
@@ -479,13 +519,15 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             em_.line(f"if (!tm_wemit(&{lo}[{ei}], &{cw}[{ei}], (double){v}, {lit(s.scale, np.float64)})) {{ "
                      f"atomicAdd(&TM_STATS[3], 1); ((u32*)P.p[{r_scr[k]}] + {3 * s.S})[{ei}] = 1u; }}")
         elif s.dtype == C.F32:
-            if k in priv:
+            if k in d64:
+                em_.line(f"atomicAdd(&tm_sh{k}[{copy_of(ei, ncopy[k])}], (double){v});")
+            elif k in priv:
                 em_.line(f"tm_ladd_f32(&tm_sh{k}[{ei}], {v});")
             else:
                 em_.line(f"tm_gadd_f32(&((float*)P.p[{r_out[k]}])[{ei}], {v});")
         elif s.dtype == C.F64:
             if k in priv:
-                em_.line(f"tm_ladd_f64(&tm_sh{k}[{ei}], {v});")
+                em_.line(f"tm_ladd_f64(&tm_sh{k}[{copy_of(ei, ncopy[k])}], {v});")
             else:
                 em_.line(f"tm_gadd_f64(&((double*)P.p[{r_out[k]}])[{ei}], {v});")
         elif s.dtype in (C.I32, C.U32):
@@ -990,9 +1032,10 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ tm_wsh{k}[i] = 0ull; "
                         f"tm_wsc{k}[i] = 0; }}")
         else:
-            ct = ctype(s.dtype)
-            body.append(f"  __shared__ {ct} tm_sh{k}[{s.S}];")
-            body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) tm_sh{k}[i] = ({ct})0;")
+            ct = "double" if k in d64 else ctype(s.dtype)
+            n = s.S * ncopy.get(k, 1)
+            body.append(f"  __shared__ {ct} tm_sh{k}[{n}];")
+            body.append(f"  for (int i = threadIdx.x; i < {n}; i += blockDim.x) tm_sh{k}[i] = ({ct})0;")
     body.append("//TM_COUNT_DECLS")
     for i in staged:
         a = bav[i]
@@ -1207,7 +1250,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         for b in range(s.S):
             if s.dtype == C.F32:
                 ldecl.append(f"  float tm_r{k}_{b} = 0.0f;")
-                body.append(f"  if (tm_r{k}_{b} != 0.0f) tm_ladd_f32(&tm_sh{k}[{b}], tm_r{k}_{b});")
+                add = f"atomicAdd(&tm_sh{k}[{copy_of(b, ncopy[k])}], (double)tm_r{k}_{b})" if k in d64 else (
+                    f"tm_ladd_f32(&tm_sh{k}[{b}], tm_r{k}_{b})")
+                body.append(f"  if (tm_r{k}_{b} != 0.0f) {add};")
             else:
                 ldecl.append(f"  {ct} tm_r{k}_{b} = 0;")
                 body.append(f"  if (tm_r{k}_{b} != 0) atomicAdd(&tm_sh{k}[{b}], tm_r{k}_{b});")
@@ -1217,7 +1262,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             counts[key] = (f"tm_cn{k}_{len(counts)}", c)
         for b, nm in enumerate(names):
             ldecl.append(f"  u32 {nm} = 0u;")
-            body.append(f"  if ({nm} != 0u) atomicAdd(&{counts[key][0]}[{b}], (u64){nm});")
+            body.append(f"  if ({nm} != 0u) atomicAdd(&{counts[key][0]}[{copy_of(b, copies(prog.tallies[k].S, LDS_F64))}], (u64){nm});")
     body[body.index("//TM_LANE_DECLS")] = "\n".join(ldecl)
     if priv:
         body.append("  __syncthreads();")
@@ -1240,18 +1285,18 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                             f"const i32 c = tm_wsc{k}[i]; if (x != 0ull) tm_wadd(&{glo}[i], &{gc}[i], (i64)x); "
                             f"if (c != 0) atomicAdd(&{gc}[i], c); }}")
             elif s.dtype == C.F64:
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const double x = tm_sh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const double x = {sum_copies(f'tm_sh{k}', ncopy[k])}; "
                             f"if (x != 0.0) tm_gadd_f64(&((double*)P.p[{r_out[k]}])[i], x); }}")
             elif s.dtype in (C.I64, C.U64):
                 ct = ctype(s.dtype)
                 body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const {ct} x = tm_sh{k}[i]; "
                             f"if (x != 0) tm_gadd_u64(&((u64*)P.p[{r_out[k]}])[i], (u64)x); }}")
             elif s.dtype == C.F32:
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const float x = tm_sh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const float x = (float){sum_copies(f'tm_sh{k}', ncopy.get(k, 1))}; "
                             f"if (x != 0.0f) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], x); }}")
                 for (kk, _), (nm, c) in counts.items():
                     if kk == k:
-                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const u64 n = {nm}[i]; "
+                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const u64 n = {sum_copies(nm, copies(s.S, LDS_F64))}; "
                                     f"if (n != 0ull) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], "
                                     f"tm_u64_f32(n) * {lit(c, np.float32)}); }}")
             else:
@@ -1262,6 +1307,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     cdecl = []
     for (k, _), (nm, c) in counts.items():
         S = prog.tallies[k].S
+        S *= copies(S, LDS_F64)
         cdecl.append(f"  __shared__ u64 {nm}[{S}];")
         cdecl.append(f"  for (int i = threadIdx.x; i < {S}; i += blockDim.x) {nm}[i] = 0ull;")
     body[body.index("//TM_COUNT_DECLS")] = "\n".join(cdecl)
