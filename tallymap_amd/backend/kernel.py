@@ -3,10 +3,10 @@
 Buffers (one by-value struct of pointers, TmParams; the item count is a kernel argument, so one code object serves
 every N):
     inputs  [per-item operands][broadcast operands]
-    results [sum tallies][exact scratch of each exact tally][ctl u32[8]][stats i32[5]] | [per-item results]
+    results [sum tallies][exact scratch of each exact tally][ctl u32][stats i32[5]] | [per-item results]
 The first group of results (up to stats) is zeroed by tm_zero before tm_main runs: the reference's n_zero
-(reference backends/kernel/kernel.py:565-591, shim.cc:215-218).  ctl holds the claim counter (u64, words 0-1) and
-the count of truncated items (word 2).
+(reference backends/kernel/kernel.py:565-591, shim.cc:215-218).  ctl holds the count of truncated items
+(word 2) and the claim counters of the item ranges.
 
 tm_main is the hand-written CDNA4 loop (reference kernel.py:812-838 is the CUDA one it replaces):
   * a persistent grid (256 CUs x achieved occupancy), block BLOCK = 256 (4 wave64s);
@@ -46,8 +46,10 @@ REG_BINS = 2               # privatised tallies of at most this many bins accumu
 XW = 9                     # int64 words per exact bin (tm_device.h TM_XW: weights 2^(32 j))
 CHUNK = 64
 RESERVE = 4                # chunks a wave reserves per claim while far from the end (short items)
-CLAIM_NS = 50              # reserve when a chunk lasted less than this many ns per resident wave (claims from every
-                           # wave at that pace would take a quarter of the counter's ~83M claims/s)
+CLAIM_NS = 20_000          # reserve when a chunk lasted less than this many ns
+SHARDS = 64                # item ranges with a claim counter each (one per lane of the wave that looks for items left)
+SHARD0 = 64                # ctl word of the first range's counter (u64), SHARD_WORDS words apart (256 bytes)
+SHARD_WORDS = 64
 COMPACT = 16               # iterations between the tail-phase repacks of a workgroup's live items
 POST_BATCH = 2.0           # finished items wait for their POST until the wave's waiting lane-iterations reach this
                            # many times the (POST + refill) / step cost ratio x 64 (0: each item's POST at once) ...
@@ -384,11 +386,11 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         rec_info.append(dict(name=rn, capacity=cap, ctr=j, fields=fl, ki=ks[0], kk=ks[1], count=prog.counts[j],
                              fin=None))
     Q = getattr(prog, "spawn", None)
-    # ctl: the item claim counter (words 0-1), truncations (word 2); a spawning program's ticket counter sits at
+    # ctl: truncations (word 2), the claim counters of the item ranges (from word SHARD0); a spawning program's ticket counter sits at
     # words 32-33, on its own 128-byte line (two counters that every wave hits serialise on a shared line), and
     # tm_qnext's generation state after it: the next generation's item count (words 40-41), children spawned and
     # dropped so far (42-43, 44-45), the roots' truncations (word 48)
-    n_ctl = 64 if Q is not None else 8
+    n_ctl = SHARD0 + SHARDS * SHARD_WORDS
     r_ctl = result((n_ctl,), np.uint32)
     r_stats = result((5,), np.int32)
     n_zero = len(res)
@@ -773,7 +775,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                        a.shape, a.dtype)
         return Val([f"(({'const ' + ct}*)P.p[{i}])[tm_item * {n} + {e}]" for e in range(n)], a.shape, a.dtype)
 
-    decls, pre_lines, step_lines, post_lines = [], [], [], []
+    decls, pre_lines, step_lines, post_lines, tail_lines = [], [], [], [], []
     pb_h = 0
 
     def write_ys(vals, trunc_idx):
@@ -866,47 +868,54 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         pb_h = int(round(float(post_batch or 0) * 64 * fin_c / max(1, step_c)))
         if pb_h < POST_BATCH_MIN:
             pb_h = 0
-        # ---- one step: cond; body or post
-        em.lines, em.ind = [], 3
-        pr = em.run(we.params["cond_jaxpr"], [sval(v) for v in cc_v] + cars)[0]
-        em.open(f"if ({pr.el[0]})")
-        bouts = em.run(we.params["body_jaxpr"], [sval(v) for v in bc_v] + cars)
-        assign_carries(em, cars, bouts)
-        em.close("} else {")
-        em.ind += 1
-        if pb_h:
+        def post():
+            """the item's POST and its per-item results."""
+            penv = {}
+            for v in jx.invars[:nT]:
+                penv[v.id] = env[v.id]
+            for v in jx.invars[nT + nP:]:
+                penv[v.id] = env[v.id]
+            for vid, x in state.items():
+                penv[vid] = x
+            for o, c in zip(we.outvars, cars):
+                penv[o.id] = c
+            for e in post_e:
+                vals = [em.value_of(penv, x) for x in e.invars]
+                for o, x in zip(e.outvars, em.eqn(e, vals)):
+                    penv[o.id] = x
+            outv = [em.value_of(penv, v) for v in jx.outvars]
+            for ln in write_ys(outv[nT:], prog.trunc):
+                em.line(ln)
+
+        def step(ind, deferred):
+            """one step of a live lane: cond; body, or the item's end (deferred: its POST waits)."""
+            em.lines, em.ind = [], ind
+            pr = em.run(we.params["cond_jaxpr"], [sval(v) for v in cc_v] + cars)[0]
+            em.open(f"if ({pr.el[0]})")
+            bouts = em.run(we.params["body_jaxpr"], [sval(v) for v in bc_v] + cars)
+            assign_carries(em, cars, bouts)
+            em.close("} else {")
+            em.ind += 1
+            if not deferred:
+                post()
             em.line("tm_live = false;")
-            em.line("tm_pend = true;")
+            if deferred:
+                em.line("tm_pend = true;")
             em.close()
-            step_lines = em.lines
-            em.lines, em.ind = [], 6
-        penv = {}
-        for v in jx.invars[:nT]:
-            penv[v.id] = env[v.id]
-        for v in jx.invars[nT + nP:]:
-            penv[v.id] = env[v.id]
-        for vid, x in state.items():
-            penv[vid] = x
-        for o, c in zip(we.outvars, cars):
-            penv[o.id] = c
-        for e in post_e:
-            vals = [em.value_of(penv, x) for x in e.invars]
-            for o, x in zip(e.outvars, em.eqn(e, vals)):
-                penv[o.id] = x
-        outv = [em.value_of(penv, v) for v in jx.outvars]
-        for ln in write_ys(outv[nT:], prog.trunc):
-            em.line(ln)
+            return em.lines
+        step_lines = step(4, pb_h > 0)
         if pb_h:
+            em.lines, em.ind = [], 7
+            post()
             post_lines = em.lines
-        else:
-            em.line("tm_live = false;")
-            em.close()
-            step_lines = em.lines
+        if compact:
+            tail_lines = step(5, False)
 
     # ------------------------------------------------------------------------------------ assemble
     from . import compile as Cm
     src = [Cm.prelude(), f"struct TmParams {{ void* p[{R}]; }};",
-           f"#define TM_STATS ((i32*)P.p[{r_stats}])", f"#define TM_CTL ((u32*)P.p[{r_ctl}])"]
+           f"#define TM_STATS ((i32*)P.p[{r_stats}])", f"#define TM_CTL ((u32*)P.p[{r_ctl}])",
+           f"#define TM_BLOCK {block}u"]
     if int(grid_cap) > 0:
         src.append(f"extern \"C\" __constant__ int tm_grid_cap = {int(grid_cap)};")
     zero_words = []
@@ -974,17 +983,20 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                    "  const i64 g = (i64)blockIdx.x * blockDim.x + threadIdx.x, st = (i64)gridDim.x * blockDim.x;\n  "
                    + "\n  ".join(post) + "\n}")
     if Q is not None:
-        # tm_qnext, one thread between two generations: the next generation's item count min(tickets, Q), the
+        # tm_qnext, one wave between two generations: the next generation's item count min(tickets, Q), the
         # spawned / dropped totals and the stats they give (children_truncated: truncations past the roots'), and
         # the claim and ticket counters cleared.  `first` (after the roots' launch) keeps the roots' truncations.
         big = 2 ** 31 - 1
         src.append("extern \"C\" __global__ void tm_qnext(const TmParams P, const i64 first) {\n"
-                   "  if (blockIdx.x != 0 || threadIdx.x != 0) return;\n"
+                   "  if (blockIdx.x != 0) return;\n"
+                   f"  for (u32 i = threadIdx.x; i < {SHARDS}u; i += blockDim.x) "
+                   f"((u64*)P.p[{r_ctl}])[{SHARD0 // 2} + i * {SHARD_WORDS // 2}u] = 0ull;\n"
+                   "  if (threadIdx.x != 0) return;\n"
                    f"  u64* const c = (u64*)P.p[{r_ctl}];\n"
                    f"  const u64 cnt = c[16], n = cnt < {Q}ull ? cnt : {Q}ull;\n"
                    "  if (first) TM_CTL[48] = TM_CTL[2];\n"
                    "  const u64 sp = c[21] + n, dr = c[22] + (cnt - n);\n"
-                   "  c[20] = n; c[21] = sp; c[22] = dr; c[0] = 0ull; c[16] = 0ull;\n"
+                   "  c[20] = n; c[21] = sp; c[22] = dr; c[16] = 0ull;\n"
                    f"  TM_STATS[0] = (i32)(sp < {big}ull ? sp : {big}ull);\n"
                    f"  TM_STATS[1] = (i32)(dr < {big}ull ? dr : {big}ull);\n"
                    "  TM_STATS[2] = (i32)(TM_CTL[2] - TM_CTL[48]);\n"
@@ -1000,6 +1012,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     lb = f"{block}, {max(1, int(min_blocks) * block // 256)}" if min_blocks else f"{block}"
     body.append(f"extern \"C\" __global__ void __launch_bounds__({lb}) {entry}(const TmParams P, "
                 f"const i64 {'tm_n_arg' if Q is not None else 'n_items'}) {{")
+    # (the grid size is read once, as a scalar, before any branch: the compiler may otherwise merge its address out of
+    # divergent prologue branches and take the whole claim control for divergent -- 94 -> 110 VGPRs in the random walk)
+    body.append("  const u32 tm_grid = tm_bcast_first(gridDim.x);")
     body.append("  u64* const tm_ctr = (u64*)P.p[%d];" % r_ctl)
     if Q is not None:          # a later generation (tm_n_arg < 0) takes its item count from tm_qnext's word
         body.append(f"  const i64 n_items = tm_n_arg >= 0 ? tm_n_arg : (i64)(tm_ctr[20] < {Q}ull ? tm_ctr[20] : {Q}ull);")
@@ -1009,7 +1024,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append(f"  __shared__ u32 tm_rleft{j}[{w}];")
         body.append(f"  if ((threadIdx.x & 63u) == 0u) {{ tm_rbase{j}[threadIdx.x >> 6] = 0ull; "
                     f"tm_rcnt{j}[threadIdx.x >> 6] = 0ull; tm_rleft{j}[threadIdx.x >> 6] = 0u; }}")
-        body.append(f"  const u64 tm_rawcap{j} = {ri['capacity']}ull + (u64)gridDim.x * {w}ull * (TM_RB - 1ull);")
+        body.append(f"  const u64 tm_rawcap{j} = {ri['capacity']}ull + (u64)tm_grid * {w}ull * (TM_RB - 1ull);")
     if Q is not None:          # the spawn ticket counter; each wave's staging rows and their count
         body.append("  u64* const tm_qctr = tm_ctr + 16;")
         if QS:
@@ -1024,24 +1039,24 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             nw = XW * s.S
             body.append(f"  __shared__ u64 tm_xsh{k}[{nw}];")
             body.append(f"  __shared__ u32 tm_xfl{k}[{(s.S + 31) // 32}];")
-            body.append(f"  for (int i = threadIdx.x; i < {nw}; i += blockDim.x) tm_xsh{k}[i] = 0ull;")
-            body.append(f"  for (int i = threadIdx.x; i < {(s.S + 31) // 32}; i += blockDim.x) tm_xfl{k}[i] = 0u;")
+            body.append(f"  for (int i = threadIdx.x; i < {nw}; i += TM_BLOCK) tm_xsh{k}[i] = 0ull;")
+            body.append(f"  for (int i = threadIdx.x; i < {(s.S + 31) // 32}; i += TM_BLOCK) tm_xfl{k}[i] = 0u;")
         elif s.fixed:
             body.append(f"  __shared__ u64 tm_wsh{k}[{s.S}];")
             body.append(f"  __shared__ i32 tm_wsc{k}[{s.S}];")
-            body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ tm_wsh{k}[i] = 0ull; "
+            body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ tm_wsh{k}[i] = 0ull; "
                         f"tm_wsc{k}[i] = 0; }}")
         else:
             ct = "double" if k in d64 else ctype(s.dtype)
             n = s.S * ncopy.get(k, 1)
             body.append(f"  __shared__ {ct} tm_sh{k}[{n}];")
-            body.append(f"  for (int i = threadIdx.x; i < {n}; i += blockDim.x) tm_sh{k}[i] = ({ct})0;")
+            body.append(f"  for (int i = threadIdx.x; i < {n}; i += TM_BLOCK) tm_sh{k}[i] = ({ct})0;")
     body.append("//TM_COUNT_DECLS")
     for i in staged:
         a = bav[i]
         ct = ctype(a.dtype)
         body.append(f"  __shared__ {ct} tm_tab{i}[{a.size}];")
-        body.append(f"  for (int i = threadIdx.x; i < {a.size}; i += blockDim.x) "
+        body.append(f"  for (int i = threadIdx.x; i < {a.size}; i += TM_BLOCK) "
                     f"tm_tab{i}[i] = ((const {ct}*)P.p[{nP + i}])[i];")
     if priv or staged:
         body.append("  __syncthreads();")
@@ -1067,10 +1082,19 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("  bool tm_live = false, tm_more = true;")
     body.append("  i64 tm_item = 0;")
     body.append("  u32 tm_loc = 0;")
-    body.append("  u64 tm_cb = 0, tm_cur = 0, tm_end = 0;     // the wave's chunk: base, next unassigned, end")
+    body.append("  u64 tm_cb = 0;                             // the wave's chunk: base item, next unassigned, end")
+    body.append("  u32 tm_cur = 0u, tm_end = 0u;")
     body.append("  u64 tm_rv = 0, tm_re = 0;                  // the wave's reservation of chunks: next, end")
     body.append("  u64 tm_t0 = 0;                             // the real-time counter at the wave's last claim")
     body.append("  u32 tm_rc = 1u;                            // chunks in the wave's last reservation")
+    body.append(f"  const u32 tm_wid = blockIdx.x * {wpb}u + tm_bcast_first(threadIdx.x >> 6);")
+    body.append(f"  const bool tm_one = (u64)n_items <= (u64)tm_grid * {wpb * chunk}u;      // at most a chunk per wave")
+    body.append("  // the ranges: counters, items per range (whole chunks), the wave's range, its items left, waves per range")
+    body.append(f"  u64* const tm_shc = tm_ctr + {SHARD0 // 2};")
+    body.append(f"  const u64 tm_shn = (((u64)n_items + {SHARDS * chunk - 1}u) / {SHARDS * chunk}u) * {chunk}u;")
+    body.append(f"  u32 tm_sh = blockIdx.x % {SHARDS}u;")
+    body.append("  u64 tm_left = tm_shn;")
+    body.append(f"  const u64 tm_shw = (tm_grid * {wpb}u + {SHARDS - 1}u) / {SHARDS}u;")
     body.append("  i32 tm_drop = 0;")
     body.append("  u32 tm_ntr = 0;")
     if pb_h:
@@ -1084,8 +1108,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("  __shared__ u32 tm_ndr;                   // waves of this workgroup whose queue is drained")
         body.append("  if (threadIdx.x == 0) { tm_pn[0] = 0u; tm_pn[1] = 0u; tm_ndr = 0u; }")
         body.append("  __syncthreads();")
-        body.append("  bool tm_dr = false, tm_bm = false;         // drained (counted), repack mode")
-        body.append("  u32 tm_it = 0, tm_round = 0;")
+        body.append("  bool tm_dr = false;                      // drained (counted)")
+        body.append("  u32 tm_round = 0;")
     body.append("  while (true) {")
     body.append("    if (tm_more) {")
     free_ = "(!tm_live && !tm_pend)" if pb_h else "!tm_live"
@@ -1095,34 +1119,58 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                     "tm_ballot(tm_live) == 0ull)) {")
     else:
         body.append("      if (tm_need != 0ull) {")
-    # one counter that every wave hits serves ~83M claims/s on MI355X, which short items at 64 per claim reach.  A
-    # wave that used up its last reservation in less than CLAIM_NS ns per resident wave per chunk (the pace at
-    # which the waves together would take a quarter of the counter's rate) reserves RESERVE chunks per claim while
-    # more than that many items per resident wave remain past its last claim; long items, and every wave's first
-    # claim, take single chunks, so their tail balances as before.  The pace is read from the 100 MHz real-time
-    # counter at claims only.
+    # Claims.  One address serves ~83M returning atomics/s (12 ns each), which short items at 64 per claim reach and
+    # which a launch's first claims (one per resident wave, up to 8,192) queue up for ~100 us at.  The items are
+    # split into SHARDS contiguous ranges, each with a counter on its own 256-byte line; a wave claims from its home
+    # range (workgroup index % SHARDS: a workgroup's XCD is its index % 8, so a range stays on one XCD and its L2)
+    # and, once that is used up, from the next range that has items left, found with one load of all counters
+    # (a lane each).  A wave learns that no items are left from one such load.  A launch of at most one chunk per
+    # wave claims nothing: wave w takes chunk w.
+    # A wave that used up its last reservation in less than CLAIM_NS ns reserves RESERVE chunks per claim while its
+    # range has more than that many chunks left per wave: a claim is a ~1 us round trip that the whole wave waits
+    # for.  The pace is read from the 100 MHz real-time counter at claims only.
     resv = chunk * RESERVE
     body.append("        if (tm_cur >= tm_end) {")
-    body.append("          if (tm_rv >= tm_re) {")
+    body.append("          if (tm_rv >= tm_re && tm_one) {")
+    body.append(f"            tm_rv = (u64)tm_wid * {chunk}u;")
+    body.append(f"            tm_re = tm_rv + {chunk}u < (u64)n_items ? tm_rv + {chunk}u : (u64)n_items;")
+    body.append("          } else if (tm_rv >= tm_re) {")
     body.append("            const u64 tm_now = __builtin_amdgcn_s_memrealtime();")
-    body.append(f"            const u64 tm_wv = (u64)gridDim.x * {wpb}u;")
-    body.append(f"            const bool tm_big = tm_t0 != 0ull && (tm_now - tm_t0) * 10ull < tm_wv * tm_rc * {CLAIM_NS}ull "
-                f"&& (u64)n_items > tm_re + tm_wv * {resv}ull;")
+    body.append(f"            const bool tm_big = tm_t0 != 0ull && (tm_now - tm_t0) * 10ull < tm_rc * {CLAIM_NS}ull "
+                f"&& tm_left > tm_shw * {resv}ull;")
     body.append(f"            tm_rc = tm_big ? {RESERVE}u : 1u;")
     body.append("            tm_t0 = tm_now;")
-    body.append(f"            tm_rv = tm_claim(tm_ctr, tm_rc * {chunk}u);")
-    body.append(f"            tm_re = tm_rv + tm_rc * {chunk}u < (u64)n_items ? tm_rv + tm_rc * {chunk}u : (u64)n_items;")
+    body.append("            while (true) {")
+    body.append("              const u64 tm_sb = tm_shn * tm_sh < (u64)n_items ? tm_shn * tm_sh : (u64)n_items;")
+    body.append("              const u64 tm_sl = tm_sb + tm_shn < (u64)n_items ? tm_shn : (u64)n_items - tm_sb;")
+    body.append(f"              const u64 tm_b = tm_claim(tm_shc + tm_sh * {SHARD_WORDS // 2}u, tm_rc * {chunk}u);")
+    body.append("              if (tm_b < tm_sl) {")
+    body.append("                tm_rv = tm_sb + tm_b;")
+    body.append(f"                tm_re = tm_sb + (tm_b + tm_rc * {chunk}u < tm_sl ? tm_b + tm_rc * {chunk}u : tm_sl);")
+    body.append("                tm_left = tm_sb + tm_sl - tm_re;")
+    body.append("                break;")
+    body.append("              }")
+    body.append("              const u64 tm_lb = tm_shn * (u64)tm_lane() < (u64)n_items ? tm_shn * (u64)tm_lane() : (u64)n_items;")
+    body.append("              const u64 tm_ll = tm_lb + tm_shn < (u64)n_items ? tm_shn : (u64)n_items - tm_lb;")
+    body.append(f"              const u64 tm_lv = __hip_atomic_load(tm_shc + tm_lane() * {SHARD_WORDS // 2}, "
+                "__ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);")
+    body.append("              const u64 tm_sm = tm_ballot(tm_lv < tm_ll);")
+    body.append("              if (tm_sm == 0ull) { tm_rv = (u64)n_items; tm_re = tm_rv; break; }")
+    body.append("              const u64 tm_hi = tm_ballot(tm_lv < tm_ll && (u32)tm_lane() >= tm_sh);   // the next from this one on")
+    body.append("              tm_sh = (u32)__builtin_ctzll(tm_hi != 0ull ? tm_hi : tm_sm);")
+    body.append("              tm_rc = 1u;")
+    body.append("            }")
     body.append("          }")
     body.append("          const u64 tm_b = tm_rv;")
     body.append("          if (tm_b >= (u64)n_items) {")
     body.append("            tm_more = false;")
     body.append("          } else {")
-    body.append(f"            tm_cb = tm_b; tm_cur = tm_b; tm_end = tm_b + {chunk}u < tm_re ? tm_b + {chunk}u : tm_re;")
-    body.append("            tm_rv = tm_end;")
+    body.append(f"            tm_cb = tm_b; tm_cur = 0u; tm_end = (u32)(tm_b + {chunk}u < tm_re ? {chunk}ull : tm_re - tm_b);")
+    body.append("            tm_rv = tm_b + tm_end;")
     if W:
         body.append(f"            for (u32 q = (u32)tm_lane(); q < {chunk}u; q += 64u) {{")
         body.append("              const u64 t = tm_cb + q;")
-        body.append("              if (t < tm_end) {")
+        body.append("              if (q < tm_end) {")
         for i, off in stage_off.items():
             n = max(1, pav[i].size)
             for e in range(n):
@@ -1133,13 +1181,13 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("          }")
     body.append("        }")
     body.append("        if (tm_cur < tm_end) {")
-    body.append("          const u64 tm_av = tm_end - tm_cur;")
-    body.append("          const u64 tm_n = (u64)__builtin_popcountll(tm_need);")
+    body.append("          const u32 tm_av = tm_end - tm_cur;")
+    body.append("          const u32 tm_n = (u32)__builtin_popcountll(tm_need);")
     body.append(f"          if ({free_}) {{")
-    body.append("            const u64 tm_r = tm_rank(tm_need);")
+    body.append("            const u32 tm_r = tm_rank(tm_need);")
     body.append("            if (tm_r < tm_av) {")
-    body.append("              tm_item = (i64)(tm_cur + tm_r);")
-    body.append("              tm_loc = (u32)(tm_cur + tm_r - tm_cb);")
+    body.append("              tm_loc = tm_cur + tm_r;")
+    body.append("              tm_item = (i64)(tm_cb + tm_loc);")
     body.append("              tm_live = true;")
     body += pre_lines
     if mode == "item":
@@ -1147,20 +1195,21 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("            }")
     body.append("          }")
     body.append("          tm_cur += tm_n < tm_av ? tm_n : tm_av;")
-    body.append("          if (tm_cur >= tm_end && tm_end >= (u64)n_items) tm_more = false;")
+    body.append("          if (tm_cur >= tm_end && (tm_one || tm_cb + tm_end >= (u64)n_items)) tm_more = false;")
     body.append("        }")
     body.append("      }")
     body.append("    }")
-    # One exit, wave-uniform (a ballot), and no `continue`: every lane reaches the claim block above on every
-    # iteration.  A per-lane `continue` lets the compiler's loop structurizer park idle lanes off the exec mask
+    # Steps until a lane is free while items are left (one step once none are): the refill's bookkeeping stays out of
+    # long items' inner loop.  Wave-uniform exits only (ballots) and no `continue`, so every lane reaches the claim
+    # block together: a per-lane `continue` lets the compiler's loop structurizer park idle lanes off the exec mask
     # while live lanes run the header again, and the claim and operand staging would then run with a partial wave.
-    body.append("    if (tm_live) {")
+    body.append("    do {")
+    body.append("      if (tm_live) {")
     body += step_lines
-    body.append("    }")
+    body.append("      }")
     if pb_h:
         # the waiting items' POST: once the wave's waiting lane-iterations reach pb_h, when no lane of the wave is
         # live, or once the queue is drained (then in the step they finish: the tail phase repacks live lanes only)
-        body.append("    {")
         body.append("      const u64 tm_pm = tm_ballot(tm_pend);")
         body.append("      if (tm_pm != 0ull) {")
         body.append("        tm_acc += (u32)__builtin_popcountll(tm_pm);")
@@ -1172,57 +1221,60 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("          }")
         body.append("        }")
         body.append("      }")
-        body.append("    }")
+    if mode == "step" and refill > 1:
+        body.append(f"    }} while (tm_more && __builtin_popcountll(tm_ballot({free_})) < {int(refill)} && "
+                    "tm_ballot(tm_live) != 0ull);")
+    else:
+        body.append(f"    }} while (tm_more && tm_ballot({free_}) == 0ull);")
     if not compact_on:
         body.append("    if (tm_ballot(tm_live || tm_more) == 0ull) break;")
+        body.append("  }")
     else:
         # Tail phase.  Every wave counts itself once when its queue is drained; when all are, the workgroup's waves
-        # repack every `compact` iterations (a wave without live lanes goes straight to the next round and waits at
-        # its barrier).  A round: live lanes write their item's loop state to the pool, barrier, every wave reads
-        # the count P (the same for all), P == 0 ends the loop for the whole workgroup, else wave w takes pool items
-        # 64 w .. 64 w + 63, barrier.  The two counters alternate: round r counts into tm_pn[r & 1] and clears the
-        # other, whose last readers finished before this round's first barrier.  Every wave runs the same number of
-        # rounds, and the loop has no other exit.
-        body.append("    if (!tm_more && !tm_dr) {")
-        body.append("      tm_dr = true;")
-        body.append("      if (tm_lane() == 0u) atomicAdd(&tm_ndr, 1u);")
+        # leave the claim loop and repack every `compact` iterations (a wave without live lanes goes straight to the
+        # next round and waits at its barrier).  A round: live lanes write their item's loop state to the pool,
+        # barrier, every wave reads the count P (the same for all), P == 0 ends the loop for the whole workgroup,
+        # else wave w takes pool items 64 w .. 64 w + 63, barrier.  The two counters alternate: round r counts into
+        # tm_pn[r & 1] and clears the other, whose last readers finished before this round's first barrier.  Every
+        # wave runs the same number of rounds, and the loop has no other exit.
+        body.append("    if (!tm_more) {")
+        body.append("      if (!tm_dr) {")
+        body.append("        tm_dr = true;")
+        body.append("        if (tm_lane() == 0u) atomicAdd(&tm_ndr, 1u);")
+        body.append("      }")
+        body.append(f"      if (__builtin_amdgcn_readfirstlane(__atomic_load_n(&tm_ndr, __ATOMIC_RELAXED)) == {wpb}u) break;")
         body.append("    }")
-        body.append("    if (tm_dr && !tm_bm) {")
-        body.append(f"      if (__builtin_amdgcn_readfirstlane(__atomic_load_n(&tm_ndr, __ATOMIC_RELAXED)) == {wpb}u) {{")
-        body.append("        tm_bm = true;")
-        body.append("        tm_it = 0u;")
+        body.append("  }")
+        body.append("  while (true) {")
+        body.append("    u32* const tm_cnt = &tm_pn[tm_round & 1u];")
+        body.append("    const u64 tm_lm = tm_ballot(tm_live);")
+        body.append("    u32 tm_pb = 0u;")
+        body.append("    if (tm_lane() == 0u) tm_pb = atomicAdd(tm_cnt, (u32)__builtin_popcountll(tm_lm));")
+        body.append("    tm_pb = __builtin_amdgcn_readfirstlane(tm_pb);")
+        body.append("    if (tm_live) {")
+        body.append("      const u32 q = tm_pb + (u32)tm_rank(tm_lm);")
+        body += ["      " + ln for ln in pack]
+        body.append("      tm_live = false;")
+        body.append("    }")
+        body.append("    __syncthreads();")
+        body.append("    const u32 tm_P = __builtin_amdgcn_readfirstlane(*tm_cnt);")
+        body.append("    if (tm_P == 0u) break;")
+        body.append("    if (threadIdx.x == 0) tm_pn[(tm_round + 1u) & 1u] = 0u;")
+        body.append("    {")
+        body.append("      const u32 q = threadIdx.x;")
+        body.append("      if (q < tm_P) {")
+        body += ["        " + ln for ln in unpack]
+        body.append("        tm_live = true;")
         body.append("      }")
         body.append("    }")
-        body.append("    if (tm_bm) {")
-        body.append("      if (tm_it == 0u || tm_ballot(tm_live) == 0ull) {")
-        body.append("        u32* const tm_cnt = &tm_pn[tm_round & 1u];")
-        body.append("        const u64 tm_lm = tm_ballot(tm_live);")
-        body.append("        u32 tm_pb = 0u;")
-        body.append("        if (tm_lane() == 0u) tm_pb = atomicAdd(tm_cnt, (u32)__builtin_popcountll(tm_lm));")
-        body.append("        tm_pb = __builtin_amdgcn_readfirstlane(tm_pb);")
-        body.append("        if (tm_live) {")
-        body.append("          const u32 q = tm_pb + (u32)tm_rank(tm_lm);")
-        body += ["          " + ln for ln in pack]
-        body.append("          tm_live = false;")
-        body.append("        }")
-        body.append("        __syncthreads();")
-        body.append("        const u32 tm_P = __builtin_amdgcn_readfirstlane(*tm_cnt);")
-        body.append("        if (tm_P == 0u) break;")
-        body.append("        if (threadIdx.x == 0) tm_pn[(tm_round + 1u) & 1u] = 0u;")
-        body.append("        {")
-        body.append("          const u32 q = threadIdx.x;")
-        body.append("          if (q < tm_P) {")
-        body += ["            " + ln for ln in unpack]
-        body.append("            tm_live = true;")
-        body.append("          }")
-        body.append("        }")
-        body.append("        __syncthreads();")
-        body.append("        ++tm_round;")
-        body.append(f"        tm_it = {compact}u;")
+        body.append("    __syncthreads();")
+        body.append("    ++tm_round;")
+        body.append(f"    for (u32 tm_it = 0u; tm_it < {compact}u && tm_ballot(tm_live) != 0ull; ++tm_it) {{")
+        body.append("      if (tm_live) {")
+        body += tail_lines
         body.append("      }")
-        body.append("      --tm_it;")
         body.append("    }")
-    body.append("  }")
+        body.append("  }")
     if QS:                     # the wave's staged children that are left
         body.append("  {")
         body.append("    const u32 tm_sq = tm_qn[threadIdx.x >> 6];")
@@ -1240,7 +1292,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append(f"    if (tm_c) atomicAdd(&((u64*)P.p[{r_rctr}])[{2 * j + 1}], tm_c);")
         body.append(f"    {fin}[1 + 2 * tm_w] = tm_c ? tm_b + (TM_RB - tm_l) : 0ull;")
         body.append(f"    {fin}[2 + 2 * tm_w] = tm_c ? tm_b + TM_RB : 0ull;")
-        body.append(f"    if (tm_w == 0) {fin}[0] = (u64)gridDim.x * {w};")
+        body.append(f"    if (tm_w == 0) {fin}[0] = (u64)tm_grid * {w};")
         body.append("  }")
     body.append("  if (tm_ntr) atomicAdd(&TM_CTL[2], tm_ntr);")
     ldecl = []
@@ -1272,36 +1324,36 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 nw = XW * s.S
                 gw = f"((u64*)P.p[{r_scr[k]}])"
                 gf = f"((u32*)P.p[{r_scr[k]}] + {2 * XW * s.S})"
-                body.append(f"  for (int i = threadIdx.x; i < {nw}; i += blockDim.x) {{ const i64 x = (i64)tm_xsh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {nw}; i += TM_BLOCK) {{ const i64 x = (i64)tm_xsh{k}[i]; "
                             f"if (x != 0 && tm_xadd(&{gw}[i / {XW} * {XW}], i % {XW}, x)) "
                             f"atomicOr(&{gf}[(i / {XW}) >> 5], 1u << ((i / {XW}) & 31)); }}")
-                body.append(f"  for (int i = threadIdx.x; i < {(s.S + 31) // 32}; i += blockDim.x) "
+                body.append(f"  for (int i = threadIdx.x; i < {(s.S + 31) // 32}; i += TM_BLOCK) "
                             f"if (tm_xfl{k}[i]) atomicOr(&{gf}[i], tm_xfl{k}[i]);")
             elif s.fixed:
                 # a block's copy: its low word added with the carry it makes, plus the block's own carries
                 glo = f"((u64*)P.p[{r_scr[k]}])"
                 gc = f"((i32*)P.p[{r_scr[k]}] + {2 * s.S})"
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const u64 x = tm_wsh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const u64 x = tm_wsh{k}[i]; "
                             f"const i32 c = tm_wsc{k}[i]; if (x != 0ull) tm_wadd(&{glo}[i], &{gc}[i], (i64)x); "
                             f"if (c != 0) atomicAdd(&{gc}[i], c); }}")
             elif s.dtype == C.F64:
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const double x = {sum_copies(f'tm_sh{k}', ncopy[k])}; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const double x = {sum_copies(f'tm_sh{k}', ncopy[k])}; "
                             f"if (x != 0.0) tm_gadd_f64(&((double*)P.p[{r_out[k]}])[i], x); }}")
             elif s.dtype in (C.I64, C.U64):
                 ct = ctype(s.dtype)
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const {ct} x = tm_sh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {ct} x = tm_sh{k}[i]; "
                             f"if (x != 0) tm_gadd_u64(&((u64*)P.p[{r_out[k]}])[i], (u64)x); }}")
             elif s.dtype == C.F32:
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const float x = (float){sum_copies(f'tm_sh{k}', ncopy.get(k, 1))}; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const float x = (float){sum_copies(f'tm_sh{k}', ncopy.get(k, 1))}; "
                             f"if (x != 0.0f) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], x); }}")
                 for (kk, _), (nm, c) in counts.items():
                     if kk == k:
-                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const u64 n = {sum_copies(nm, copies(s.S, LDS_F64))}; "
+                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const u64 n = {sum_copies(nm, copies(s.S, LDS_F64))}; "
                                     f"if (n != 0ull) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], "
                                     f"tm_u64_f32(n) * {lit(c, np.float32)}); }}")
             else:
                 ct = ctype(s.dtype)
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += blockDim.x) {{ const {ct} x = tm_sh{k}[i]; "
+                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {ct} x = tm_sh{k}[i]; "
                             f"if (x != 0) atomicAdd(&(({ct}*)P.p[{r_out[k]}])[i], x); }}")
     body.append("}")
     cdecl = []
@@ -1309,7 +1361,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         S = prog.tallies[k].S
         S *= copies(S, LDS_F64)
         cdecl.append(f"  __shared__ u64 {nm}[{S}];")
-        cdecl.append(f"  for (int i = threadIdx.x; i < {S}; i += blockDim.x) {nm}[i] = 0ull;")
+        cdecl.append(f"  for (int i = threadIdx.x; i < {S}; i += TM_BLOCK) {nm}[i] = 0ull;")
     body[body.index("//TM_COUNT_DECLS")] = "\n".join(cdecl)
     src.append("\n".join(body))
     aux = []
