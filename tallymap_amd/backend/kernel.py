@@ -26,6 +26,7 @@ import numpy as np
 
 from .. import _core as C
 from .codegen import Emitter, Val, VTally, assign_carries, ctype, lit
+from . import ahead as Ahead
 from . import simplify
 
 BLOCK = 256
@@ -50,6 +51,8 @@ CLAIM_NS = 20_000          # reserve when a chunk lasted less than this many ns
 SHARDS = 64                # item ranges with a claim counter each (one per lane of the wave that looks for items left)
 SHARD0 = 64                # ctl word of the first range's counter (u64), SHARD_WORDS words apart (256 bytes)
 SHARD_WORDS = 64
+SPREAD = 16                # lanes per item a small launch of a program with steps computed ahead spreads to (the
+                           # launcher's grid, the module's tm_spread)
 COMPACT = 16               # iterations between the tail-phase repacks of a workgroup's live items
 POST_BATCH = 2.0           # finished items wait for their POST until the wave's waiting lane-iterations reach this
                            # many times the (POST + refill) / step cost ratio x 64 (0: each item's POST at once) ...
@@ -467,6 +470,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     rcounts = {}                # the same, for a lane-register tally: -> (the lane's u32 counter names per bin, value)
 
     quiet = set(getattr(prog, "quiet_tallies", ()))
+    lead = [False]              # emitting the update side of a group of lanes (tail loop)
 
     def emit_rule(em_, e, ins):
         t, idx, val = ins
@@ -475,13 +479,15 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         if s.kind == "discard":
             return t
         ei = em_.bind(idx.el[0], np.int32, "ei")
-        if k in quiet:
-            em_.open(f"if ((u32){ei} < {s.S}u)")
+        ok = em_.bind(f"(u32){ei} < {s.S}u", C.BOOL, "ok")
+        if lead[0]:            # (a group of lanes holds the item: one of them emits)
+            if k not in quiet:
+                em_.line(f"tm_drop += (tm_lead && !{ok}) ? 1 : 0;")
+            em_.open(f"if (tm_lead && {ok})")
         else:
-            em_.open(f"if ((u32){ei} >= {s.S}u)")
-            em_.line("++tm_drop;")
-            em_.close("} else {")
-            em_.ind += 1
+            if k not in quiet:
+                em_.line(f"tm_drop += {ok} ? 0 : 1;")
+            em_.open(f"if ({ok})")
         v = val.el[0]
         lv = e.invars[2]
         if k in rpriv:
@@ -612,7 +618,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         W, ck = int(e.params["words"]), bool(e.params.get("ck", False))
         ws = [w_ for v in ins[3:] for w_ in _words_of(em_, v)]
         ws += ["0u"] * (W - len(ws))
-        em_.open(f"if ((u32)({k.el[0]}) {'==' if ck else '<'} (u32)({cap.el[0]}))")
+        em_.open(f"if ({'tm_lead && ' if lead[0] else ''}(u32)({k.el[0]}) {'==' if ck else '<'} (u32)({cap.el[0]}))")
         p = tape_row(em_, k.el[0], cap.el[0], "", ck)
         u = 4 if W % 4 == 0 else (2 if W % 2 == 0 else 1)
         for q in range(0, W, u):
@@ -624,23 +630,10 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         return t
     em.hooks["tallymap_tape_put"] = tape_put_rule
 
-    def tape_get_rule(em_, e, ins):
-        """the leaves stored in slot j (< cap) of the item's tape row, or (ck) in its checkpoint."""
-        j, cap = ins
-        W, ck = int(e.params["words"]), bool(e.params.get("ck", False))
-        p = tape_row(em_, j.el[0], cap.el[0], "const ", ck)
-        words = []
-        u = 4 if W % 4 == 0 else (2 if W % 2 == 0 else 1)
-        for q in range(0, W, u):
-            if u == 1:
-                words.append(em_.bind(f"{p}[{q}]", C.U32, "tq"))
-                continue
-            v = em_.fresh("tq")
-            em_.line(f"const tm_u32x{u} {v} = *(const tm_u32x{u}*)&{p}[{q}];")
-            words += [f"{v}.{c}" for c in "xyzw"[:u]]
+    def _vals_of(em_, words, avals):
+        """the values of `avals` whose elements' u32 words are `words` (_words_of's order)."""
         outs, w_ = [], 0
-        for o in e.outvars:
-            a = o.aval
+        for a in avals:
             ct = ctype(a.dtype)
             els = []
             for _ in range(max(1, a.size)):
@@ -659,6 +652,22 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                     w_ += 1
             outs.append(Val(els, a.shape, a.dtype))
         return outs
+
+    def tape_get_rule(em_, e, ins):
+        """the leaves stored in slot j (< cap) of the item's tape row, or (ck) in its checkpoint."""
+        j, cap = ins
+        W, ck = int(e.params["words"]), bool(e.params.get("ck", False))
+        p = tape_row(em_, j.el[0], cap.el[0], "const ", ck)
+        words = []
+        u = 4 if W % 4 == 0 else (2 if W % 2 == 0 else 1)
+        for q in range(0, W, u):
+            if u == 1:
+                words.append(em_.bind(f"{p}[{q}]", C.U32, "tq"))
+                continue
+            v = em_.fresh("tq")
+            em_.line(f"const tm_u32x{u} {v} = *(const tm_u32x{u}*)&{p}[{q}];")
+            words += [f"{v}.{c}" for c in "xyzw"[:u]]
+        return _vals_of(em_, words, [o.aval for o in e.outvars])
     em.hooks["tallymap_tape_get"] = tape_get_rule
 
     def spawn_rule(em_, e, ins):
@@ -776,7 +785,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         return Val([f"(({'const ' + ct}*)P.p[{i}])[tm_item * {n} + {e}]" for e in range(n)], a.shape, a.dtype)
 
     decls, pre_lines, step_lines, post_lines, tail_lines = [], [], [], [], []
-    pb_h = 0
+    pb_h, pl_ahead = 0, None
 
     def write_ys(vals, trunc_idx):
         lines = []
@@ -908,14 +917,60 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             em.lines, em.ind = [], 7
             post()
             post_lines = em.lines
+        def tail_ahead(pl):
+            """a group's round in the tail loop (Ahead): lane tm_go of the group computes the values of the step
+            tm_go ahead, then the group runs tm_g updates, update j on the values of its lane j."""
+            bj, nb_ = we.params["body_jaxpr"], we.params["body_nconsts"]
+            em.lines, em.ind = [], 4
+            ins_ = [sval(v) for v in bc_v] + cars
+            e_ = {v.id: x for v, x in zip(bj.invars, ins_)}
+            for j, gain in pl.counters.items():
+                v = bj.invars[nb_ + j]
+                e_[v.id] = Val([em.bind(f"({ctype(v.aval.dtype)})((u32){cars[j].el[0]} + tm_go * {gain & 0xffffffff}u)",
+                                        v.aval.dtype, "kg")], (), v.aval.dtype)
+            for q in pl.ahead:
+                for o, x in zip(q.outvars, em.eqn(q, [em.value_of(e_, v) for v in q.invars])):
+                    e_[o.id] = x
+            words = [w_ for v in pl.cut for w_ in _words_of(em, e_[v.id])]
+            for i, w_ in enumerate(words):
+                em.line(f"tm_h{i} = {w_};")
+            head = em.lines
+            em.lines, em.ind = [], 4
+            lead[0] = True
+            # (the condition on every lane, an item's end under a wave-uniform branch: one lane mask per update)
+            pr = em.run(we.params["cond_jaxpr"], [sval(v) for v in cc_v] + cars)[0]
+            em.line(f"const bool tm_go_on = tm_live && {pr.el[0]};")
+            em.open("if (tm_ballot(tm_live && !tm_go_on) != 0ull)")
+            em.open("if (tm_live && !tm_go_on && tm_lead)")
+            lead[0] = False
+            post()
+            lead[0] = True
+            em.close()
+            em.line("tm_live = tm_go_on;")
+            em.close()
+            em.open("if (tm_go_on)")
+            e_ = {v.id: x for v, x in zip(bj.invars, ins_)}
+            for v, x in zip(pl.cut, _vals_of(em, [f"tm_q{i}" for i in range(len(words))], [v.aval for v in pl.cut])):
+                e_[v.id] = x
+            for q in pl.update:
+                for o, x in zip(q.outvars, em.eqn(q, [em.value_of(e_, v) for v in q.invars])):
+                    e_[o.id] = x
+            assign_carries(em, cars, [em.value_of(e_, v) for v in bj.outvars])
+            lead[0] = False
+            em.close()
+            return head, em.lines, len(words)
         if compact:
-            tail_lines = step(5, False)
+            pl_ahead = Ahead.plan(we, lambda v: isinstance(v, C.Var) and isinstance(env.get(v.id), VTally), cost) \
+                if Q is None and not recs else None
+            tail_lines = tail_ahead(pl_ahead) if pl_ahead is not None else step(5, False)
 
     # ------------------------------------------------------------------------------------ assemble
     from . import compile as Cm
     src = [Cm.prelude(), f"struct TmParams {{ void* p[{R}]; }};",
            f"#define TM_STATS ((i32*)P.p[{r_stats}])", f"#define TM_CTL ((u32*)P.p[{r_ctl}])",
            f"#define TM_BLOCK {block}u"]
+    if pl_ahead:
+        src.append(f"extern \"C\" __constant__ int tm_spread = {SPREAD};")
     if int(grid_cap) > 0:
         src.append(f"extern \"C\" __constant__ int tm_grid_cap = {int(grid_cap)};")
     zero_words = []
@@ -1089,6 +1144,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("  u32 tm_rc = 1u;                            // chunks in the wave's last reservation")
     body.append(f"  const u32 tm_wid = blockIdx.x * {wpb}u + tm_bcast_first(threadIdx.x >> 6);")
     body.append(f"  const bool tm_one = (u64)n_items <= (u64)tm_grid * {wpb * chunk}u;      // at most a chunk per wave")
+    # (with steps computed ahead, a wave takes an even share: few items per workgroup are many lanes per item)
+    body.append(f"  const u32 tm_ch = (u32)(((u64)n_items + tm_grid * {wpb}u - 1u) / (tm_grid * {wpb}u));"
+                if pl_ahead else f"  const u32 tm_ch = {chunk}u;")
     body.append("  // the ranges: counters, items per range (whole chunks), the wave's range, its items left, waves per range")
     body.append(f"  u64* const tm_shc = tm_ctr + {SHARD0 // 2};")
     body.append(f"  const u64 tm_shn = (((u64)n_items + {SHARDS * chunk - 1}u) / {SHARDS * chunk}u) * {chunk}u;")
@@ -1109,6 +1167,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("  if (threadIdx.x == 0) { tm_pn[0] = 0u; tm_pn[1] = 0u; tm_ndr = 0u; }")
         body.append("  __syncthreads();")
         body.append("  bool tm_dr = false;                      // drained (counted)")
+        if pl_ahead:
+            body.append("  bool tm_lead = true;                     // (tail) the lane of its item's group that emits")
         body.append("  u32 tm_round = 0;")
     body.append("  while (true) {")
     body.append("    if (tm_more) {")
@@ -1132,8 +1192,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     resv = chunk * RESERVE
     body.append("        if (tm_cur >= tm_end) {")
     body.append("          if (tm_rv >= tm_re && tm_one) {")
-    body.append(f"            tm_rv = (u64)tm_wid * {chunk}u;")
-    body.append(f"            tm_re = tm_rv + {chunk}u < (u64)n_items ? tm_rv + {chunk}u : (u64)n_items;")
+    body.append("            tm_rv = (u64)tm_wid * tm_ch;")
+    body.append("            tm_re = tm_rv + tm_ch < (u64)n_items ? tm_rv + tm_ch : (u64)n_items;")
     body.append("          } else if (tm_rv >= tm_re) {")
     body.append("            const u64 tm_now = __builtin_amdgcn_s_memrealtime();")
     body.append(f"            const bool tm_big = tm_t0 != 0ull && (tm_now - tm_t0) * 10ull < tm_rc * {CLAIM_NS}ull "
@@ -1247,21 +1307,26 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("  }")
         body.append("  while (true) {")
         body.append("    u32* const tm_cnt = &tm_pn[tm_round & 1u];")
-        body.append("    const u64 tm_lm = tm_ballot(tm_live);")
+        body.append(f"    const u64 tm_lm = tm_ballot(tm_live{' && tm_lead' if pl_ahead else ''});")
         body.append("    u32 tm_pb = 0u;")
         body.append("    if (tm_lane() == 0u) tm_pb = atomicAdd(tm_cnt, (u32)__builtin_popcountll(tm_lm));")
         body.append("    tm_pb = __builtin_amdgcn_readfirstlane(tm_pb);")
-        body.append("    if (tm_live) {")
+        body.append("    if (tm_live && tm_lead) {" if pl_ahead else "    if (tm_live) {")
         body.append("      const u32 q = tm_pb + (u32)tm_rank(tm_lm);")
         body += ["      " + ln for ln in pack]
-        body.append("      tm_live = false;")
         body.append("    }")
+        body.append("    tm_live = false;")
         body.append("    __syncthreads();")
         body.append("    const u32 tm_P = __builtin_amdgcn_readfirstlane(*tm_cnt);")
         body.append("    if (tm_P == 0u) break;")
         body.append("    if (threadIdx.x == 0) tm_pn[(tm_round + 1u) & 1u] = 0u;")
+        if pl_ahead:
+            body.append("    u32 tm_gs = 0u;")
+            body.append("    while (tm_gs < 6u && (tm_P << (tm_gs + 1u)) <= TM_BLOCK) ++tm_gs;")
+            body.append("    const u32 tm_g = 1u << tm_gs, tm_go = (u32)tm_lane() & (tm_g - 1u);")
+            body.append("    tm_lead = tm_go == 0u;")
         body.append("    {")
-        body.append("      const u32 q = threadIdx.x;")
+        body.append("      const u32 q = threadIdx.x >> tm_gs;" if pl_ahead else "      const u32 q = threadIdx.x;")
         body.append("      if (q < tm_P) {")
         body += ["        " + ln for ln in unpack]
         body.append("        tm_live = true;")
@@ -1269,11 +1334,33 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("    }")
         body.append("    __syncthreads();")
         body.append("    ++tm_round;")
-        body.append(f"    for (u32 tm_it = 0u; tm_it < {compact}u && tm_ballot(tm_live) != 0ull; ++tm_it) {{")
-        body.append("      if (tm_live) {")
-        body += tail_lines
-        body.append("      }")
-        body.append("    }")
+        if pl_ahead is None:
+            body.append(f"    for (u32 tm_it = 0u; tm_it < {compact}u && tm_ballot(tm_live) != 0ull; ++tm_it) {{")
+            body.append("      if (tm_live) {")
+            body += tail_lines
+            body.append("      }")
+            body.append("    }")
+        else:
+            # Groups of tm_g lanes hold an item each (a power of two, 1 .. 64, from the items left), every lane of a
+            # group with the same state; one of them emits and writes.  With at most an item per wave left a round
+            # ends with the wave's item.  The cross-lane reads (ds_bpermute, the next update's issued before this
+            # one's work) stand outside any lane-dependent branch: all lanes of the wave are active there.
+            head, upd, nw = tail_lines
+            body.append(f"    const u32 tm_nb = tm_P <= {wpb}u ? ~0u : ({compact}u >> tm_gs) + ({compact}u >> tm_gs == 0u ? 1u : 0u);")
+            body.append("    const int tm_ba = (int)(((u32)tm_lane() & ~(tm_g - 1u)) * 4u);")
+            body.append("    for (u32 tm_it = 0u; tm_it < tm_nb && tm_ballot(tm_live) != 0ull; ++tm_it) {")
+            body += [f"      u32 tm_h{i} = 0u;" for i in range(nw)]
+            body.append("      if (tm_live) {")
+            body += head
+            body.append("      }")
+            body += [f"      u32 tm_n{i} = (u32)__builtin_amdgcn_ds_bpermute(tm_ba, (int)tm_h{i});" for i in range(nw)]
+            body.append("      for (u32 tm_j = 1u; tm_j <= tm_g && tm_ballot(tm_live) != 0ull; ++tm_j) {")
+            body += [f"        const u32 tm_q{i} = tm_n{i};" for i in range(nw)]
+            body += [f"        tm_n{i} = (u32)__builtin_amdgcn_ds_bpermute(tm_ba + (int)((tm_j & (tm_g - 1u)) * 4u), "
+                     f"(int)tm_h{i});" for i in range(nw)]
+            body += upd
+            body.append("      }")
+            body.append("    }")
         body.append("  }")
     if QS:                     # the wave's staged children that are left
         body.append("  {")

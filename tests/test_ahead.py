@@ -1,0 +1,84 @@
+"""What backend/ahead.py takes out of a step: only values that depend on the step through its counters, and every value
+the rest of the step reads is one it has."""
+import numpy as np
+import pytest
+
+from tallymap_amd import _core as C
+from tallymap_amd import configs, lax, problems, random
+from tallymap_amd import numpy as jnp
+from tallymap_amd._api import Sum, build_program
+from tallymap_amd.backend import ahead as A
+from tallymap_amd.backend import kernel as K
+
+
+def _plan(item, outputs, axes, args, max_steps=None):
+    pav = [C.AVal(np.shape(a)[1:], np.asarray(a).dtype) for a, x in zip(args, axes) if x == 0]
+    bav = [C.AVal(np.shape(a), np.asarray(a).dtype) for a, x in zip(args, axes) if x is None]
+    prog, _ = build_program(item, outputs, axes, pav, bav, max_steps)
+    we = prog.jaxpr.eqns[K._split(prog.jaxpr)]
+    tallies = {v.id for v in prog.jaxpr.invars[:prog.nT]}
+    for e in prog.jaxpr.eqns:           # (a tally stays one through emits)
+        if e.prim == "tallymap_emit" and e.invars[0].id in tallies:
+            tallies.add(e.outvars[0].id)
+    return A.plan(we, lambda v: isinstance(v, C.Var) and v.id in tallies, K.cost), we
+
+
+def _sound(pl, we):
+    """the update side reads only loop operands, its own results and the cut; the ahead side only loop constants,
+    counters, carries that never change and its own results; together they hold every equation."""
+    bj, nb = we.params["body_jaxpr"], we.params["body_nconsts"]
+    have = {v.id for v in bj.invars} | {v.id for v in pl.cut}
+    for e in pl.update:
+        assert all(v.id in have for v in e.invars if isinstance(v, C.Var)), e
+        have |= {o.id for o in e.outvars}
+    assert all(v.id in have for v in bj.outvars if isinstance(v, C.Var))
+    same = {v.id for v, o in zip(bj.invars[nb:], bj.outvars) if isinstance(o, C.Var) and o.id == v.id}
+    have = {v.id for v in bj.invars[:nb]} | same | {bj.invars[nb + j].id for j in pl.counters}
+    for e in pl.ahead:
+        assert A._pure(e)
+        assert all(v.id in have for v in e.invars if isinstance(v, C.Var)), e
+        have |= {o.id for o in e.outvars}
+    assert {id(e) for e in pl.ahead} | {id(e) for e in pl.update} == {id(e) for e in bj.eqns}
+
+
+@pytest.mark.parametrize("name, words", [("c1", 1), ("c2", 1), ("c3", 9), ("c4", 2), ("random_walk", 2),
+                                         ("transport", 4), ("walk_on_spheres", 6), ("barrier", 1), ("gillespie", 2)])
+def test_programs_that_draw(name, words):
+    cfg = getattr(configs, name.upper(), None) or problems.PROBLEMS[name]
+    args = cfg["inputs"](8)[0] if "inputs" in cfg else getattr(configs, name + "_inputs")(8)
+    pl, we = _plan(cfg["item"], cfg["outputs"], cfg["in_axes"], args, cfg.get("max_steps"))
+    _sound(pl, we)
+    assert sum(max(1, v.aval.size) for v in pl.cut) <= words
+
+
+@pytest.mark.parametrize("name", ["c5", "ode_ensemble"])
+def test_programs_without_draws_have_no_plan(name):
+    cfg = getattr(configs, name.upper(), None) or problems.PROBLEMS[name]
+    args = cfg["inputs"](8)[0] if "inputs" in cfg else getattr(configs, name + "_inputs")(8)
+    assert _plan(cfg["item"], cfg["outputs"], cfg["in_axes"], args, cfg.get("max_steps"))[0] is None
+
+
+def _walk(draw):
+    """a walk whose draw is draw(key, k, x, m) -> (u, the next m)."""
+    def item(t, x, key):
+        def body(c):
+            k, x, m, t = c
+            u, m = draw(key, k, x, m)
+            return k + 1, x * (0.5 + 0.5 * u), m, t.add("h", (x * 4).astype(jnp.int32), u)
+        k, x, m, t = lax.while_loop(lambda c: c[1] > 0.05, body, (np.int32(0), x, np.int32(7), t))
+        return t, k
+    return _plan(item, {"h": Sum((4,))}, (0, 0), (np.ones(2, np.float32), np.zeros((2, 2), np.uint32)))
+
+
+def test_what_counts_as_a_counter():
+    u = random.uniform
+    for gain in (1, -3, 5):             # any literal gain
+        pl, we = _walk(lambda key, k, x, m: (u(random.fold_in(key, m)), m + gain))
+        _sound(pl, we)
+        assert gain in pl.counters.values()
+    pl, we = _walk(lambda key, k, x, m: (u(random.fold_in(key, k)) + m.astype(jnp.float32), m))     # never changes
+    _sound(pl, we)
+    # a gain that is not a literal, or a draw keyed by the state: nothing to compute ahead
+    assert _walk(lambda key, k, x, m: (u(random.fold_in(key, m)), m + k))[0] is None
+    assert _walk(lambda key, k, x, m: (u(random.fold_in(key, m)), m * 2))[0] is None
+    assert _walk(lambda key, k, x, m: (u(random.fold_in(key, (x * 100).astype(jnp.int32))), m + 1))[0] is None
