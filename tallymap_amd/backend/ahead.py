@@ -24,7 +24,7 @@ from . import simplify
 
 MIN_COST = 64              # instructions (kernel.cost) the ahead part has to save per step: about one hash
 MAX_WORDS = 16             # 32-bit words that pass per step (a register and a cross-lane read each)
-PURE = simplify.PURE | {"tallymap_item_index"}
+PURE = simplify.PURE | {"tallymap_item_index", "tallymap_sincos"}
 
 
 @dataclasses.dataclass
@@ -35,9 +35,10 @@ class Plan:
     counters: dict         # carry index -> its gain per step
 
 
-def _pure(e):
+def pure(e):
+    """whether e computes values alone (no tally, tape, queue or record effect)."""
     if e.prim in ("while", "cond"):
-        return all(_pure(x) for j in C.subjaxprs(e) for x in j.eqns)
+        return all(pure(x) for j in C.subjaxprs(e) for x in j.eqns)
     return e.prim in PURE or (not C.subjaxprs(e) and not e.prim.startswith("tallymap_"))
 
 
@@ -76,7 +77,7 @@ def plan(we, is_tally, cost):
     ahead, update = [], []
     for e in bj.eqns:
         ks = {kind[v.id] for v in e.invars if isinstance(v, C.Var)}
-        if "update" in ks or not _pure(e):
+        if "update" in ks or not pure(e):
             k = "update"
         elif ks <= {"inv"}:
             k = "inv"

@@ -143,6 +143,8 @@ class Emitter:
         # branch after another, so wave-shared LDS state must not pass between branches through plain loads and
         # first-lane stores (the kernel assembler's spawn and Records rules read it)
         self.div = 0
+        # element expressions known once per kernel -> the name of their float64 reciprocal (set by the kernel assembler)
+        self.invariant = {}
 
     # -------------------------------------------------------------------------------- text helpers
     def fresh(self, p="t"):
@@ -371,6 +373,8 @@ def _ew(em, e, ins):
     out = e.outvars[0].aval
     t = ctype(out.dtype)
     n = max(1, out.size)
+    if e.prim == "div" and t == "float":
+        return _div_f32(em, e, ins, n)
     rule = EW[e.prim]
     # the operation's type: the operands' (a comparison's result is bool)
     it = ctype(e.invars[0].aval.dtype)
@@ -379,6 +383,28 @@ def _ew(em, e, ins):
     for i in range(n):
         args = [_bc(x, i, n) for x in ins]
         res.append(em.bind(rule(at, args), out.dtype))
+    return Val(res, out.shape, out.dtype)
+
+
+def _div_f32(em, e, ins, n):
+    """float32 division: by the float64 reciprocal where the divisor is known before the loop (tm_div_by) -- a literal,
+    or a value computed once per kernel (Emitter.invariant) -- else the correctly rounded division."""
+    out = e.outvars[0].aval
+    y = e.invars[1]
+    lits = None
+    if isinstance(y, C.Lit):
+        lits = [float(x) for x in np.asarray(y.val, np.float32).reshape(-1)]
+    res = []
+    for i in range(n):
+        a, b = _bc(ins[0], i, n), _bc(ins[1], i, n)
+        inv = None
+        if lits is not None:
+            v = lits[0] if len(lits) == 1 else lits[i]
+            if np.isfinite(v) and v != 0.0 and abs(np.frexp(v)[0]) != 0.5:     # (a power of two: an exact product)
+                inv = lit(1.0 / v, np.float64)
+        else:
+            inv = em.invariant.get(b)
+        res.append(em.bind(f"({a} / {b})" if inv is None else f"tm_div_by({a}, {b}, {inv})", out.dtype))
     return Val(res, out.shape, out.dtype)
 
 
@@ -515,6 +541,20 @@ def _ct_read(em, e, ins):
     S = max(1, int(np.prod(arr.shape)))
     i = idx.el[0]
     return Val([em.bind(f"((u32)({i}) < {S}u ? {arr.ptr}[{i}] : 0.0f)", C.F32, "ct")], (), C.F32)
+
+
+@rule("tallymap_sincos")
+def _sincos(em, e, ins):
+    """sin and cos of one operand (simplify.pair_sincos)."""
+    a = e.outvars[0].aval
+    ss, cs = [], []
+    for x in ins[0].el:
+        s, c = em.fresh("sn"), em.fresh("cs")
+        em.line(f"float {s}, {c};")
+        em.line(f"tm_sincosf({x}, {s}, {c});")
+        ss.append(s)
+        cs.append(c)
+    return [Val(ss, a.shape, a.dtype), Val(cs, a.shape, a.dtype)]
 
 
 @rule("threefry2x32")

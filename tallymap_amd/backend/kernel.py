@@ -148,7 +148,7 @@ def _free_vars(jx):
 
 
 _HEAVY = {"exp", "log", "sin", "cos", "tan", "atan", "atan2", "asin", "acos", "sinh", "cosh", "tanh", "asinh", "acosh",
-          "atanh", "log1p", "expm1", "exp2", "log2", "pow", "erf", "erfc", "erf_inv", "lgamma", "cbrt", "logistic"}
+          "atanh", "log1p", "expm1", "exp2", "log2", "pow", "erf", "erfc", "erf_inv", "lgamma", "cbrt", "logistic", "tallymap_sincos"}
 _FREE = {"slice", "squeeze", "reshape", "broadcast_in_dim", "concatenate", "copy", "stop_gradient"}
 
 
@@ -167,7 +167,7 @@ def cost(eqns, loop=4):
             brs = [b for i, b in enumerate(e.params["branches"]) if i not in cold] or list(e.params["branches"])
             c += 2 + max(cost(b.eqns, loop) for b in brs)
         elif p in _HEAVY:
-            c += 30 * n
+            c += 30 * n * len(e.outvars)
         elif p == "threefry2x32":
             c += 72 * n
         elif p in ("div", "rem", "sqrt", "rsqrt"):
@@ -356,7 +356,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     claims and queue flushes, at the cost of latency hiding."""
     chunk = max(1, int(chunk))
     compact = max(0, int(compact))
-    jx = simplify.cse(prog.jaxpr, _split(prog.jaxpr))
+    jx = simplify.drop_draw_clamp(prog.jaxpr)
+    jx = simplify.cse(jx, _split(jx))
+    jx = simplify.pair_sincos(jx, _split(jx))
     nT, nP, nB = prog.nT, prog.nP, prog.nB
     pav, bav = prog.p_avals(), prog.b_avals()
     yav = prog.y_avals()
@@ -784,7 +786,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                        a.shape, a.dtype)
         return Val([f"(({'const ' + ct}*)P.p[{i}])[tm_item * {n} + {e}]" for e in range(n)], a.shape, a.dtype)
 
-    decls, pre_lines, step_lines, post_lines, tail_lines = [], [], [], [], []
+    decls, pre_lines, step_lines, post_lines, tail_lines, uni_lines = [], [], [], [], [], []
     pb_h, pl_ahead = 0, None
 
     def write_ys(vals, trunc_idx):
@@ -827,7 +829,36 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             env[v.id] = Val([em.bind(x, a.dtype, "x") for x in lv.el], a.shape, a.dtype)
         for v, bv in zip(jx.invars[nT + nP:], bvals):
             env[v.id] = bv
+        # PRE values of broadcast operands alone are the same for every item: computed once per kernel, held as scalars
+        # (no state per lane, nothing to repack), and their reciprocals taken there (tm_div_by)
+        loads, uni = em.lines, set(bids)
+        em.lines, em.ind = [], 1
+        once = [el for a, bv in zip(bav, bvals) if a.dtype == C.F32 and a.size <= BCAST_REG for el in bv.el]
         for e in pre_e:
+            if not Ahead.pure(e) or any(x.prim == "tallymap_item_index" for x in C.walk_eqns(C.Jaxpr([], [], [e]))) \
+                    or not all(isinstance(v, C.Lit) or v.id in uni for v in e.invars) or any(
+                    o.aval.dtype.itemsize != 4 or o.aval.size > BCAST_REG for o in e.outvars):
+                continue
+            outs_ = em.eqn(e, [em.value_of(env, x) for x in e.invars])
+            for o, x in zip(e.outvars, outs_):
+                names = []
+                for el in x.el:
+                    names.append(em.bind(f"__builtin_bit_cast({ctype(x.dtype)}, tm_bcast_first(__builtin_bit_cast(u32, "
+                                         f"({ctype(x.dtype)})({el}))))", x.dtype, "un"))
+                env[o.id] = Val(names, x.shape, x.dtype)
+                uni.add(o.id)
+                if x.dtype == C.F32:
+                    once += names
+        for i_, el in enumerate(once):
+            nm = em.invariant[el] = f"tm_rc{i_}"
+            em.line(f"const u64 {nm}u = __builtin_bit_cast(u64, 1.0 / (double){el});")
+            em.line(f"const double {nm} = __builtin_bit_cast(double, (u64)tm_bcast_first((u32){nm}u) | "
+                    f"((u64)tm_bcast_first((u32)({nm}u >> 32)) << 32));")
+        uni_lines, bids = em.lines, uni
+        em.lines, em.ind = loads, 5
+        for e in pre_e:
+            if all(o.id in uni for o in e.outvars) and e.outvars:
+                continue
             vals = [em.value_of(env, x) for x in e.invars]
             for o, x in zip(e.outvars, em.eqn(e, vals)):
                 env[o.id] = x
@@ -882,8 +913,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             penv = {}
             for v in jx.invars[:nT]:
                 penv[v.id] = env[v.id]
-            for v in jx.invars[nT + nP:]:
-                penv[v.id] = env[v.id]
+            for i_ in bids:
+                penv[i_] = env[i_]
+            penv.update((i_, x) for i_, x in env.items() if isinstance(x, VTally))     # (emitted into by PRE)
             for vid, x in state.items():
                 penv[vid] = x
             for o, c in zip(we.outvars, cars):
@@ -1121,6 +1153,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             continue
         for e in range(max(1, a.size)):
             body.append(f"  const {ct} tm_b{i}_{e} = ((const {ct}*)P.p[{nP + i}])[{e}];")
+    body += uni_lines
     wpb = block // 64
     compact_on = bool(compact) and mode == "step"
     if compact_on:

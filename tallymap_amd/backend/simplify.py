@@ -102,3 +102,102 @@ def cse(jx, cut=None):
     if not changed:
         return jx
     return C.Jaxpr(jx.invars, [r(v) for v in jx.outvars], eqns)
+
+
+def _map_subs(e, f):
+    """e with f applied to each of its sub-programs (the same equation when nothing changes)."""
+    new = {}
+    for k, p in e.params.items():
+        if isinstance(p, C.Jaxpr):
+            new[k] = f(p)
+        elif isinstance(p, (list, tuple)) and any(isinstance(x, C.Jaxpr) for x in p):
+            xs = [f(x) if isinstance(x, C.Jaxpr) else x for x in p]
+            new[k] = p if all(a is b for a, b in zip(xs, p)) else type(p)(xs)
+        else:
+            new[k] = p
+    if all(new[k] is p for k, p in e.params.items()):
+        return e
+    return C.Eqn(e.prim, e.invars, e.outvars, new)
+
+
+def pair_sincos(jx, cut=None):
+    """sin x and cos x of one float32 x in a jaxpr (on one side of `cut`) -> one tallymap_sincos equation (two results):
+    the reduction and the polynomials of the two calls are the same values, which the device compiler does not share
+    (they sit in two divergent branches).  Programs that draw a direction, and the derivatives of either function,
+    hold such pairs."""
+    eqns = [_map_subs(e, pair_sincos) for e in jx.eqns]
+    first = {}                      # x -> index of the first of the pair
+    drop = set()
+    for i, e in enumerate(eqns):
+        if i == cut:
+            first = {}
+        if e.prim not in ("sin", "cos") or e.outvars[0].aval.dtype != C.F32 or not isinstance(e.invars[0], C.Var):
+            continue
+        k = e.invars[0].id
+        j = first.setdefault(k, i)
+        if j == i or eqns[j].prim not in ("sin", "cos") or eqns[j].prim == e.prim:
+            continue
+        a, b = (eqns[j], e) if eqns[j].prim == "sin" else (e, eqns[j])
+        eqns[j] = C.Eqn("tallymap_sincos", [e.invars[0]], [a.outvars[0], b.outvars[0]], {})
+        drop.add(i)
+    if not drop and all(a is b for a, b in zip(eqns, jx.eqns)):
+        return jx
+    return C.Jaxpr(jx.invars, jx.outvars, [e for i, e in enumerate(eqns) if i not in drop])
+
+
+def drop_draw_clamp(jx):
+    """max(lo, f * span + lo) -> f * span + lo, where f = (bits >> 9 | 1.0f's bits) as a float - 1 and span >= 0
+    (jax.random.uniform's clamp): f is in [0, 1), so f * span + lo >= lo in float32 too (rounding is monotonic), never
+    -0 for lo = 0, and the max is its operand."""
+    eqns = [_map_subs(e, drop_draw_clamp) for e in jx.eqns]
+    by = {o.id: e for e in eqns for o in e.outvars}
+
+    def lit(v):
+        return float(np.asarray(v.val).reshape(-1)[0]) if isinstance(v, C.Lit) and np.asarray(v.val).size == 1 else None
+
+    def of(v, prim):
+        e = by.get(v.id) if isinstance(v, C.Var) else None
+        return e if e is not None and e.prim == prim else None
+
+    def pick(e, f):
+        """the (literal, other operand) of a binary equation with f(other) true, else (None, None)."""
+        for a, b in (e.invars, e.invars[::-1]):
+            if lit(a) is not None and isinstance(b, C.Var) and f(b):
+                return lit(a), b
+        return None, None
+
+    def unit(v):
+        """v = bitcast(shift_right_logical(bits, 9) | 0x3F800000) - 1"""
+        e = of(v, "sub")
+        e = of(e.invars[0], "bitcast_convert_type") if e is not None and lit(e.invars[1]) == 1.0 else None
+        e = of(e.invars[0], "or") if e is not None and e.outvars[0].aval.dtype == C.F32 else None
+        if e is None:
+            return False
+        c, x = pick(e, lambda b: of(b, "shift_right_logical") is not None)
+        return c == 0x3F800000 and lit(of(x, "shift_right_logical").invars[1]) == 9.0
+
+    def clamped(e):
+        """the operand that max equation e returns, or None."""
+        if e.prim != "max" or e.outvars[0].aval.dtype != C.F32 or e.outvars[0].aval.shape != ():
+            return None
+        lo, s = pick(e, lambda b: of(b, "add") is not None)
+        if lo is None or not np.isfinite(lo) or (lo == 0.0 and np.signbit(lo)):
+            return None
+        lo2, m = pick(of(s, "add"), lambda b: of(b, "mul") is not None)
+        if lo2 != lo or np.signbit(lo2) != np.signbit(lo):
+            return None
+        span, _ = pick(of(m, "mul"), unit)
+        return s if span is not None and 0.0 <= span < np.inf else None
+
+    sub, out = {}, []
+    for e in eqns:
+        if any(isinstance(v, C.Var) and v.id in sub for v in e.invars):
+            e = C.Eqn(e.prim, [sub.get(v.id, v) if isinstance(v, C.Var) else v for v in e.invars], e.outvars, e.params)
+        s = clamped(e)
+        if s is not None:
+            sub[e.outvars[0].id] = s
+            continue
+        out.append(e)
+    if not sub and all(a is b for a, b in zip(eqns, jx.eqns)):
+        return jx
+    return C.Jaxpr(jx.invars, [sub.get(v.id, v) if isinstance(v, C.Var) else v for v in jx.outvars], out)

@@ -95,10 +95,17 @@ TM_FN float tm_i64f(i64 x) {
 }
 
 // ------------------------------------------------------------------------------------------- lax helpers
+// (float32 on gfx950: v_maximum3_f32 / v_minimum3_f32 are exactly these, one instruction for the ~8 of the comparisons)
 template <class T> TM_FN T tm_fmax(T a, T b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(T) == 4) return __builtin_elementwise_maximum(a, b);
+#endif
   return (a > b || a != a) ? a : ((b > a || b != b) ? b : (a == (T)0 ? a + b : a));
 }
 template <class T> TM_FN T tm_fmin(T a, T b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(T) == 4) return __builtin_elementwise_minimum(a, b);
+#endif
   return (a < b || a != a) ? a : ((b < a || b != b) ? b : (a == (T)0 ? -(-a - b) : a));
 }
 template <class T> TM_FN T tm_imax(T a, T b) { return a > b ? a : b; }
@@ -239,7 +246,20 @@ TM_FN double tm_fmod(double x, double y) {
   return (ux >> 63) ? -v : v;
 }
 
-// float -> integer toward zero, saturating, NaN -> 0
+// float -> integer toward zero, saturating, NaN -> 0: what v_cvt_i32 / v_cvt_u32 do, written as the instruction where
+// the C conversion would be undefined out of range and the guards around it cost four compares and selects
+#if defined(__HIP_DEVICE_COMPILE__)
+#define TM_CVT32(name, R, F, ins) \
+  TM_FN R name(F x) { \
+    R r; \
+    asm(ins " %0, %1" : "=v"(r) : "v"(x)); \
+    return r; \
+  }
+TM_CVT32(tm_f2i32, i32, float, "v_cvt_i32_f32")
+TM_CVT32(tm_f2u32, u32, float, "v_cvt_u32_f32")
+TM_CVT32(tm_d2i32, i32, double, "v_cvt_i32_f64")
+TM_CVT32(tm_d2u32, u32, double, "v_cvt_u32_f64")
+#else
 TM_FN i32 tm_f2i32(float x) {
   return x != x ? 0 : (x <= -2147483648.0f ? (i32)0x80000000u : (x >= 2147483648.0f ? 0x7fffffff : (i32)x));
 }
@@ -252,6 +272,7 @@ TM_FN i32 tm_d2i32(double x) {
 TM_FN u32 tm_d2u32(double x) {
   return x != x ? 0u : (x <= 0.0 ? 0u : (x >= 4294967295.0 ? 0xffffffffu : (u32)x));
 }
+#endif
 TM_FN i64 tm_f2i64(float x) {
   return x != x ? 0 : (x <= -9223372036854775808.0f ? (i64)0x8000000000000000ull
                                                      : (x >= 9223372036854775808.0f ? 0x7fffffffffffffffll : (i64)x));
@@ -259,6 +280,17 @@ TM_FN i64 tm_f2i64(float x) {
 TM_FN i64 tm_d2i64(double x) {
   return x != x ? 0 : (x <= -9223372036854775808.0 ? (i64)0x8000000000000000ull
                                                     : (x >= 9223372036854775808.0 ? 0x7fffffffffffffffll : (i64)x));
+}
+
+// x / y in float32 with inv = 1 / y in float64: x * inv is within 2^-52 of the quotient, and a float32 quotient above
+// the smallest normal is at least 2^-49 (relative) from the midpoint of two floats -- it would take a dividend of 25
+// significant bits to be one -- so rounding the product is the correctly rounded quotient.  A result below that is
+// divided.  Infinities, NaN and zeros of either operand pass through the product, or are divided as results of 0.
+// Where y is known before the loop (a literal, a value of broadcast operands): three instructions for ~12.
+TM_FN float tm_div_by(float x, float y, double inv) {
+  float q = (float)((double)x * inv);
+  if (__builtin_expect(__builtin_fabsf(q) < 0x1p-126f, 0)) q = x / y;
+  return q;
 }
 
 // ----------------------------------------------------------------------------------------- threefry2x32

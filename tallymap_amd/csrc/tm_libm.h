@@ -260,12 +260,9 @@ TM_FN float tm_logf(float x) {
   const double A0 = -0x1.00ea348b88334p-2, A1 = 0x1.5575b0be00b6ap-2, A2 = -0x1.ffffef20a4123p-2;
   const double Ln2 = 0x1.62e42fefa39efp-1;
   u32 ix = tm_f2u(x);
-  if (ix == 0x3f800000u) return 0.0f;
-  if (ix - 0x00800000u >= 0x7f800000u - 0x00800000u) {
-    if (ix * 2u == 0u) return -__builtin_inff();
-    if (ix == 0x7f800000u) return x;
-    if ((ix & 0x80000000u) || ix * 2u >= 0xff000000u) return __builtin_nanf("");
-    ix = tm_f2u(x * 0x1p23f);                     // a subnormal: normalise
+  const bool rare = ix - 0x00800000u >= 0x7f800000u - 0x00800000u;
+  if (__builtin_expect(rare, 0)) {
+    ix = tm_f2u(x * 0x1p23f);                     // a subnormal: normalise (the others are replaced below)
     ix -= 23u << 23;
   }
   const u32 tmp = ix - 0x3f330000u;
@@ -279,7 +276,14 @@ TM_FN float tm_logf(float x) {
   double y = __builtin_fma(A1, r, A2);
   y = __builtin_fma(A0, r2, y);
   y = __builtin_fma(y, r2, y0 + r);
-  return (float)y;
+  float res = (float)y;
+  if (__builtin_expect(rare, 0)) {
+    const u32 ux = tm_f2u(x);
+    if (ux * 2u == 0u) res = -__builtin_inff();
+    else if (ux == 0x7f800000u) res = x;
+    else if ((ux & 0x80000000u) || ux * 2u >= 0xff000000u) res = __builtin_nanf("");
+  }
+  return res;
 }
 
 // ------------------------------------------------------------------------------------------------ expf
@@ -355,7 +359,7 @@ TM_FN float tm_sc_poly(double x, double x2, int n, bool flip) {
 // |x| < 120: n = round(x 2/pi) (through 2^24-scaled integer arithmetic), x - n pi/2 with one fma
 TM_FN double tm_sc_reduce_fast(double x, int* np) {
   const double r = x * TM_SC_HPI_INV;
-  const int n = ((i32)r + 0x800000) >> 24;
+  const int n = (tm_d2i32(r) + 0x800000) >> 24;    // (any x may come here; the caller replaces what |x| >= 120 gives)
   *np = n;
   return __builtin_fma(-(double)n, TM_SC_HPI, x);
 }
@@ -384,41 +388,55 @@ TM_FN u32 tm_abstop12(float x) { return (tm_f2u(x) >> 20) & 0x7ffu; }
 // n = 0 and r = y exactly, and the same polynomial: one path for every |y| < 120, so the lanes of a wave do not
 // split on |y| < pi/4, with y itself selected below 2^-12 (the polynomial turns -0 into +0).  Bitwise glibc's on
 // all 2^32 inputs.
-TM_FN float tm_sinf(float y) {
-  double x = y;
+// The rare arguments (|y| >= 120) replace the result afterwards, in a branch no wave takes in ordinary work: the common
+// path runs without a lane mask of its own.
+TM_FN float tm_sinf_large(float y) {
+  if (tm_abstop12(y) >= tm_abstop12(__builtin_inff())) return y - y;
   int n;
-  if (tm_abstop12(y) < tm_abstop12(120.0f)) {
-    x = tm_sc_reduce_fast(x, &n);
-    const double s = tm_sc_sign(n);
-    const float r = tm_sc_poly(x * s, x * x, n, (n & 2) != 0);
-    return tm_abstop12(y) < tm_abstop12(0x1p-12f) ? y : r;
-  }
-  if (tm_abstop12(y) < tm_abstop12(__builtin_inff())) {
-    const u32 xi = tm_f2u(y);
-    const int sign = (int)(xi >> 31);
-    x = tm_sc_reduce_large(xi, &n);
-    const double s = tm_sc_sign(n + sign);
-    return tm_sc_poly(x * s, x * x, n, ((n + sign) & 2) != 0);
-  }
-  return y - y;
+  const u32 xi = tm_f2u(y);
+  const double x = tm_sc_reduce_large(xi, &n);
+  const int q = n + (int)(xi >> 31);
+  return tm_sc_poly(x * tm_sc_sign(q), x * x, n, (q & 2) != 0);
+}
+TM_FN float tm_cosf_large(float y) {
+  if (tm_abstop12(y) >= tm_abstop12(__builtin_inff())) return y - y;
+  int n;
+  const u32 xi = tm_f2u(y);
+  const double x = tm_sc_reduce_large(xi, &n);
+  const int q = n + (int)(xi >> 31);
+  return tm_sc_poly(x * tm_sc_sign(q), x * x, n ^ 1, (q & 2) != 0);
+}
+TM_FN float tm_sinf(float y) {
+  int n;
+  const double x = tm_sc_reduce_fast(y, &n);
+  float r = tm_sc_poly(x * tm_sc_sign(n), x * x, n, (n & 2) != 0);
+  if (tm_abstop12(y) < tm_abstop12(0x1p-12f)) r = y;
+  if (__builtin_expect(tm_abstop12(y) >= tm_abstop12(120.0f), 0)) r = tm_sinf_large(y);
+  return r;
 }
 TM_FN float tm_cosf(float y) {             // (one path for |y| < 120, as tm_sinf; glibc returns 1 below 2^-12)
-  double x = y;
   int n;
-  if (tm_abstop12(y) < tm_abstop12(120.0f)) {
-    x = tm_sc_reduce_fast(x, &n);
-    const double s = tm_sc_sign(n);
-    const float r = tm_sc_poly(x * s, x * x, n ^ 1, (n & 2) != 0);
-    return tm_abstop12(y) < tm_abstop12(0x1p-12f) ? 1.0f : r;
+  const double x = tm_sc_reduce_fast(y, &n);
+  float r = tm_sc_poly(x * tm_sc_sign(n), x * x, n ^ 1, (n & 2) != 0);
+  if (tm_abstop12(y) < tm_abstop12(0x1p-12f)) r = 1.0f;
+  if (__builtin_expect(tm_abstop12(y) >= tm_abstop12(120.0f), 0)) r = tm_cosf_large(y);
+  return r;
+}
+// both of one angle: the reduction and the two polynomials once (tm_sinf and tm_cosf evaluate both polynomials each and
+// select).  Bitwise tm_sinf's and tm_cosf's.
+TM_FN void tm_sincosf(float y, float& sin_y, float& cos_y) {
+  int n;
+  const double x = tm_sc_reduce_fast(y, &n);
+  const double xs = x * tm_sc_sign(n), x2 = x * x;
+  const float a = tm_sc_poly(xs, x2, 0, false), c = tm_sc_poly(xs, x2, 1, (n & 2) != 0);   // sine, cosine polynomial
+  const bool tiny = tm_abstop12(y) < tm_abstop12(0x1p-12f), odd = (n & 1) != 0;
+  float rs = tiny ? y : (odd ? c : a), rc = tiny ? 1.0f : (odd ? a : c);
+  if (__builtin_expect(tm_abstop12(y) >= tm_abstop12(120.0f), 0)) {
+    rs = tm_sinf_large(y);
+    rc = tm_cosf_large(y);
   }
-  if (tm_abstop12(y) < tm_abstop12(__builtin_inff())) {
-    const u32 xi = tm_f2u(y);
-    const int sign = (int)(xi >> 31);
-    x = tm_sc_reduce_large(xi, &n);
-    const double s = tm_sc_sign(n + sign);
-    return tm_sc_poly(x * s, x * x, n ^ 1, ((n + sign) & 2) != 0);
-  }
-  return y - y;
+  sin_y = rs;
+  cos_y = rc;
 }
 
 // ----------------------------------------------------------------------------------------------------- tanf
@@ -497,19 +515,17 @@ TM_FN float tm_atanf(float x) {
     if (ix > 0x7f800000) return x + x;
     return hx > 0 ? atanhi[3] + atanlo[3] : -atanhi[3] - atanlo[3];
   }
-  if (ix < 0x3ee00000) {
-    if (ix < 0x31000000) return x;
-    id = -1;
-  } else {
-    x = __builtin_fabsf(x);
-    if (ix < 0x3f980000) {
-      if (ix < 0x3f300000) { id = 0; x = (2.0f * x - 1.0f) / (2.0f + x); }
-      else { id = 1; x = (x - 1.0f) / (x + 1.0f); }
-    } else {
-      if (ix < 0x401c0000) { id = 2; x = (x - 1.5f) / (1.0f + 1.5f * x); }
-      else { id = 3; x = -1.0f / x; }
-    }
-  }
+  if (ix < 0x31000000) return x;
+  // the four reductions' quotients as one division of selected operands (x / 1 is x): the lanes of a wave are in
+  // several ranges, and a division in each branch would run one after another
+  const float a = __builtin_fabsf(x);
+  float num, den;
+  if (ix < 0x3ee00000) { id = -1; num = x; den = 1.0f; }
+  else if (ix < 0x3f300000) { id = 0; num = 2.0f * a - 1.0f; den = 2.0f + a; }
+  else if (ix < 0x3f980000) { id = 1; num = a - 1.0f; den = a + 1.0f; }
+  else if (ix < 0x401c0000) { id = 2; num = a - 1.5f; den = 1.0f + 1.5f * a; }
+  else { id = 3; num = -1.0f; den = a; }
+  x = num / den;
   const float z = x * x, w = z * z;
   const float s1 = z * (aT[0] + w * (aT[2] + w * (aT[4] + w * (aT[6] + w * (aT[8] + w * aT[10])))));
   const float s2 = w * (aT[1] + w * (aT[3] + w * (aT[5] + w * (aT[7] + w * aT[9]))));

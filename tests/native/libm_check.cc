@@ -124,6 +124,8 @@ int main(int argc, char** argv) {
     else if (!strcmp(argv[2], "expf")) { mine = tm_expf; ref = expf; }
     else if (!strcmp(argv[2], "sinf")) { mine = tm_sinf; ref = sinf; }
     else if (!strcmp(argv[2], "cosf")) { mine = tm_cosf; ref = cosf; }
+    else if (!strcmp(argv[2], "sincosf_s")) { mine = [](float x) { float s, c; tm_sincosf(x, s, c); return s; }; ref = sinf; }
+    else if (!strcmp(argv[2], "sincosf_c")) { mine = [](float x) { float s, c; tm_sincosf(x, s, c); return c; }; ref = cosf; }
     else if (!strcmp(argv[2], "atanf")) { mine = tm_atanf; ref = atanf; }
     else if (!strcmp(argv[2], "exp2f")) { mine = tm_exp2f; ref = exp2f; }
     else if (!strcmp(argv[2], "log2f")) { mine = tm_log2f; ref = log2f; }

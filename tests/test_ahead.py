@@ -35,7 +35,7 @@ def _sound(pl, we):
     same = {v.id for v, o in zip(bj.invars[nb:], bj.outvars) if isinstance(o, C.Var) and o.id == v.id}
     have = {v.id for v in bj.invars[:nb]} | same | {bj.invars[nb + j].id for j in pl.counters}
     for e in pl.ahead:
-        assert A._pure(e)
+        assert A.pure(e)
         assert all(v.id in have for v in e.invars if isinstance(v, C.Var)), e
         have |= {o.id for o in e.outvars}
     assert {id(e) for e in pl.ahead} | {id(e) for e in pl.update} == {id(e) for e in bj.eqns}

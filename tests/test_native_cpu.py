@@ -187,7 +187,7 @@ def test_erfinv_log_absolute_error(libm):
     assert r.returncode == 0, r.stdout
 
 
-@pytest.mark.parametrize("fn", ["logf", "expf", "sinf", "cosf", "atanf", "exp2f", "log2f", "expm1f", "log1pf",
+@pytest.mark.parametrize("fn", ["logf", "expf", "sinf", "cosf", "sincosf_s", "sincosf_c", "atanf", "exp2f", "log2f", "expm1f", "log1pf",
                                 "tanhf", "logistic", "asinf", "acosf", "sinhf", "coshf", "atanhf", "asinhf",
                                 "acoshf", "erff", "erfcf", "tanf", "lgammaf"])
 def test_f32_libm_bitwise_equal_to_glibc(libm, fn):
@@ -427,6 +427,15 @@ def test_fmod_matches_glibc(tmp_path):
     assert r.returncode == 0, r.stdout
     bad, tot = map(int, r.stdout.split()[-2:])
     assert bad == 0 and tot > 8_000_000
+
+
+def test_division_by_a_reciprocal_is_the_division(tmp_path):
+    """tm_div_by: bitwise x / y on special values, random pairs, quotients next to midpoints and subnormal ones."""
+    exe = _build("tests/native/div_check.cc", str(tmp_path / "div_check"))
+    r = subprocess.run([exe, "8000000"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+    bad, tot = map(int, r.stdout.split()[-2:])
+    assert bad == 0 and tot > 32_000_000
 
 
 def test_uniform_derived_arguments_match_glibc(libm):
