@@ -19,7 +19,6 @@ from . import util as U
 _KERNELS = collections.OrderedDict()
 _LOCK = threading.Lock()
 KERNEL_CACHE = 256
-RB = 256                   # slots per Records batch (TM_RB in tm_device.h)
 
 
 @dataclasses.dataclass
@@ -147,13 +146,13 @@ def _alloc_specs(c, N):
             continue
         if per_item == "tape":          # per launched lane (the launcher's persistent grid at this N)
             sh = (_lanes(c, N),) + tuple(shape)
-        elif per_item == ("rraw",):     # a Records raw buffer: the capacity + 255 spare slots per launched wave
-            sh = (int(shape[0]) + (_lanes(c, N) // 64) * (RB - 1) if N > 0 else int(shape[0]),)
+        elif isinstance(per_item, tuple) and per_item[0] == "rraw":
+            # a Records raw buffer: the capacity and room for a partly used batch per launched wave
+            S = per_item[1]
+            sh = (S * K.raw_segment_slots(int(shape[0]), _lanes(c, N) // 64, S) if N > 0 else int(shape[0]),)
             if sh[0] > 2 ** 31 - 1:
                 raise ValueError(f"tallymap_amd: a Records capacity of {shape[0]} leaves no room for the launch's "
                                  "batch slack below 2^31 slots")
-        elif per_item == ("rwave",):    # a Records hole list: a count, then a slot range per launched wave
-            sh = (1 + 2 * (_lanes(c, N) // 64),)
         else:
             sh = ((N,) + tuple(shape)) if per_item else tuple(shape)
         outs.append((sh, torch_dtype(dt)))
@@ -174,12 +173,11 @@ def _queue(c, ins, outs, N, n_zero, flags, stream=None, n_main=None):
     Cm.check(Cm.lib().tm_launch(c.id, ctypes.c_void_p(s), arr, len(bufs), n_zero, flags,
                                 N if n_main is None else n_main, c.block))
     if n_main == 0:
-        N = 0          # (tm_main did not run: its per-wave hole lists are unwritten, so the passes see no items)
+        N = 0          # (tm_main did not run: no item has a record, so the passes see no items)
     for name, kind, block, cap in (getattr(L, "aux", None) or []):
         if N == 0 and kind != "cap":         # (no item ran: only the canonical outputs are written, as zeros)
             continue
-        grid = {"items": -(-int(N) // 1024), "one": 1, "cap": min(-(-int(cap) // 256), 4096),
-                "waves": max(1, -(-(_lanes(c, N) // 64) // 256))}[kind]
+        grid = {"items": -(-int(N) // 1024), "one": 1, "cap": min(-(-int(cap) // 256), 4096)}[kind]
         Cm.check(Cm.lib().tm_launch_aux(c.id, name.encode(), ctypes.c_void_p(s), arr, len(bufs), N, grid, block))
 
 

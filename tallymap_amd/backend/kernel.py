@@ -51,6 +51,10 @@ CLAIM_NS = 20_000          # reserve when a chunk lasted less than this many ns
 SHARDS = 64                # item ranges with a claim counter each (one per lane of the wave that looks for items left)
 SHARD0 = 64                # ctl word of the first range's counter (u64), SHARD_WORDS words apart (256 bytes)
 SHARD_WORDS = 64
+RC_WORDS = SHARDS * SHARD_WORDS + 64    # u32 words of a Records output's counters: a u64 of slots claimed per segment of
+                           # its raw slots (SHARD_WORDS apart), then (u64) the records appended and the launch's waves
+RC_TOTAL = SHARDS * SHARD_WORDS // 2    # u64 index of the records appended among them
+RB = 256                   # slots per Records batch (TM_RB in tm_device.h)
 SPREAD = 16                # lanes per item a small launch of a program with steps computed ahead spreads to (the
                            # launcher's grid, the module's tm_spread)
 COMPACT = 16               # iterations between the tail-phase repacks of a workgroup's live items
@@ -181,16 +185,16 @@ def cost(eqns, loop=4):
 
 def _records_passes(ri, r_rctr, r_out, r_cnt, r_rex, r_rbs, prog, bad):
     """the passes that move Records output j's raw records to their canonical slots (replacing the reference's
-    _records.canon, _records.py:45-74): tm_rholes<j> (the unused slots of each wave's last batch get key 0),
-    tm_rscan<j> (blocks of 1024 items: the exclusive prefix sum of the per-item counts within the block, and the
+    _records.canon, _records.py:45-74): tm_rscan<j> (blocks of 1024 items: the exclusive prefix sum of the per-item counts within the block, and the
     block's total), tm_rtop<j> (one block: the exclusive prefix sum of the block totals), tm_rcanon<j> (every claimed
     raw slot with a key: record (i, k) to slot offset[i] + k; the slots past the last record zeroed; when `bad` -- a
     truncation or any Records output past its capacity (reference _api.py:745-755) -- every float field NaN and
     every integer field -1 instead)."""
     j, cap = ri["ctr"], ri["capacity"]
     cnt, rex, rbs = f"((const i32*)P.p[{r_cnt}])", f"((i64*)P.p[{r_rex}])", f"((i64*)P.p[{r_rbs}])"
-    slots, tot = f"((const u64*)P.p[{r_rctr}])[{2 * j}]", f"((const u64*)P.p[{r_rctr}])[{2 * j + 1}]"
-    fin = f"((const u64*)P.p[{ri['fin']}])"
+    rc, S = f"((const u64*)P.p[{r_rctr}] + {RC_WORDS // 2 * j})", ri["segments"]
+    nb = f"({-(-cap // RB)}ull + {rc}[{RC_TOTAL + 1}])"          # (raw_segment_slots, with the launch's waves)
+    seg = (f"{cap}ull + {rc}[{RC_TOTAL + 1}] * {RB - 1}ull" if S == 1 else f"({nb} + {S - 1}ull) / {S}ull * {RB}ull")
     ki, kk = f"((i32*)P.p[{r_out[ri['ki']]}])", f"((const i32*)P.p[{r_out[ri['kk']]}])"
     scan = ("  for (int d = 1; d < 1024; d <<= 1) {\n"
             "    const i64 x = (int)threadIdx.x >= d ? tm_s[threadIdx.x - d] : 0;\n"
@@ -199,12 +203,6 @@ def _records_passes(ri, r_rctr, r_out, r_cnt, r_rex, r_rbs, prog, bad):
             "    __syncthreads();\n"
             "  }\n")
     out = []
-    out.append(f"extern \"C\" __global__ void __launch_bounds__(256) tm_rholes{j}(const TmParams P, const i64 n_items) {{\n"
-               f"  const u64 nw = {fin}[0], rawcap = {cap}ull + nw * (TM_RB - 1ull);\n"
-               "  for (u64 w = (u64)blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += (u64)gridDim.x * blockDim.x) {\n"
-               f"    const u64 s1 = {fin}[2 + 2 * w] < rawcap ? {fin}[2 + 2 * w] : rawcap;\n"
-               f"    for (u64 s = {fin}[1 + 2 * w]; s < s1; ++s) {ki}[s] = 0;\n"
-               "  }\n}")
     out.append(f"extern \"C\" __global__ void __launch_bounds__(1024) tm_rscan{j}(const TmParams P, const i64 n_items) {{\n"
                "  __shared__ i64 tm_s[1024];\n"
                "  const i64 i = (i64)blockIdx.x * 1024 + threadIdx.x;\n"
@@ -241,18 +239,40 @@ def _records_passes(ri, r_rctr, r_out, r_cnt, r_rex, r_rbs, prog, bad):
                f"    for (i64 s = g; s < {cap}; s += st) {{ {' '.join(fill)} }}\n"
                "    return;\n"
                "  }\n"
-               f"  const i64 nslots = (i64){slots}, ntot = (i64){tot};\n"
-               "  for (i64 s = g; s < nslots; s += st) {\n"
-               f"    const i32 key = {ki}[s];\n"
-               "    if (key <= 0 || (i64)key > n_items) continue;\n"
-               f"    const i32 cid = key - 1, k = {kk}[s];\n"
-               f"    const i64 dst = {rex}[cid] + {rbs}[cid >> 10] + k;\n"
-               f"    if (dst < 0 || dst >= {cap}) continue;\n"
-               f"    {' '.join(mv)}\n"
+               f"  const i64 ntot = (i64){rc}[{RC_TOTAL}], seg = (i64)({seg});\n"
+               # a segment's slots go to the workgroups of its index modulo the segments: on MI355X a workgroup's XCD is
+               # its index % 8, the XCD whose waves wrote the segment and whose items' records it mostly holds
+               f"  for (i64 q = blockIdx.x % {S}; q < {S}; q += gridDim.x) {{\n"
+               f"    const i64 parts = gridDim.x >= {S}u ? (i64)((gridDim.x - q + {S - 1}) / {S}) : 1;\n"
+               f"    const i64 part = gridDim.x >= {S}u ? (i64)(blockIdx.x / {S}u) : 0;\n"
+               f"    const i64 n = (i64){rc}[q * {SHARD_WORDS // 2}] < seg ? (i64){rc}[q * {SHARD_WORDS // 2}] : seg;\n"
+               "    for (i64 i = part * 256 + threadIdx.x; i < n; i += parts * 256) {\n"
+               "      const i64 s = q * seg + i;\n"
+               f"      const i32 key = {ki}[s];\n"
+               "      if (key <= 0 || (i64)key > n_items) continue;\n"
+               f"      const i32 cid = key - 1, k = {kk}[s];\n"
+               f"      const i64 dst = {rex}[cid] + {rbs}[cid >> 10] + k;\n"
+               f"      if (dst < 0 || dst >= {cap}) continue;\n"
+               f"      {' '.join(mv)}\n"
+               "    }\n"
                "  }\n"
                f"  for (i64 s = ntot + g; s < {cap}; s += st) {{ {' '.join(zero)} }}\n"
                "}")
     return "\n".join(out)
+
+
+def raw_segments(capacity, direct):
+    """segments a Records output's raw slots are split into, each with its own slot counter (1: the claims are of other
+    sizes than a batch, or the slots come near 2^31)."""
+    return 1 if direct or capacity > 2 ** 30 else SHARDS
+
+
+def raw_segment_slots(capacity, waves, S):
+    """the raw slots of a segment, for a launch of `waves` waves: room for every record of the capacity and one partly
+    used batch per wave, in whole batches per segment."""
+    if S == 1:
+        return capacity + waves * (RB - 1)
+    return RB * -(-(-(-capacity // RB) + waves) // S)
 
 
 def exact_words(S):
@@ -373,12 +393,22 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     raw = set()                # the Records outputs' raw tallies: sized per launch (capacity + the waves' batch
     for rn, _, _ in (getattr(prog, "records", ()) or ()):     # slack), never zeroed, stored to once per slot
         raw |= {k for k in outs if prog.tallies[k].name.startswith(rkey(rn, ""))}
-    r_out = {k: result(prog.tallies[k].shape, prog.tallies[k].dtype, ("rraw",) if k in raw else False)
+    # appends inside a cond claim slots one point at a time (tm_rclaim_direct): such an output keeps one segment
+    segs = {}
+    for j, (rn, cap, _) in enumerate(getattr(prog, "records", ()) or ()):
+        direct = any(x.prim == "tallymap_claim" and int(x.params["r"]) == j for e in C.walk_eqns(jx) if e.prim == "cond"
+                     for b in C.subjaxprs(e) for x in C.walk_eqns(b))
+        segs[rn] = raw_segments(int(cap), direct)
+
+    def raw_of(k):
+        """the Records output whose raw tally k is."""
+        return next(rn for rn in segs if prog.tallies[k].name.startswith(rkey(rn, "")))
+    r_out = {k: result(prog.tallies[k].shape, prog.tallies[k].dtype, ("rraw", segs[raw_of(k)]) if k in raw else False)
              for k in outs}
     r_scr = {k: result((scratch_words(prog.tallies[k]),), np.uint32) for k in outs
              if prog.tallies[k].exact or prog.tallies[k].fixed}
     recs = list(getattr(prog, "records", ()) or ())
-    r_rctr = result((4 * len(recs),), np.uint32) if recs else None     # per output: u64 slots claimed, u64 records
+    r_rctr = result((RC_WORDS * len(recs),), np.uint32) if recs else None
     rec_info = []
     for j, (rn, cap, _) in enumerate(recs):
         pre, keys = rkey(rn, ""), (rkey(rn, KI), rkey(rn, KK))
@@ -389,7 +419,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 fl[nm[len(pre):]] = (k, result((cap,), prog.tallies[k].dtype))
         ks = [k for k in outs if prog.tallies[k].name in keys]
         rec_info.append(dict(name=rn, capacity=cap, ctr=j, fields=fl, ki=ks[0], kk=ks[1], count=prog.counts[j],
-                             fin=None))
+                             segments=segs[rn]))
     Q = getattr(prog, "spawn", None)
     # ctl: truncations (word 2), the claim counters of the item ranges (from word SHARD0); a spawning program's ticket counter sits at
     # words 32-33, on its own 128-byte line (two counters that every wave hits serialise on a shared line), and
@@ -412,8 +442,6 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     QS = (128 if q_words <= 16 else 64 if q_words <= 48 else 0) if Q is not None else 0
     r_rex = result((), np.int64, per_item=True) if recs else None       # the Records scans' scratch (per item)
     r_rbs = result((), np.int64, per_item=True) if recs else None
-    for ri in rec_info:        # per launched wave: the unused slot range [s0, s1) of its last batch (+ a count)
-        ri["fin"] = result((), np.uint64, per_item=("rwave",))
     # the tape adjoint's programs (backend/tape.py): a u32 buffer of N x cap x Wp words (cap: an operand), written
     # by the count program's tape puts and read by the reverse program's gets; the caller allocates it
     tape_w = int(getattr(prog, "tape_words", 0) or 0)
@@ -567,11 +595,12 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         t, w, _ = ins
         j = int(e.params["r"])
         if em_.div:
-            sl = em_.bind(f"(i32)tm_rclaim_direct(&((u64*)P.p[{r_rctr}])[{2 * j}], "
+            sl = em_.bind(f"(i32)tm_rclaim_direct((u64*)P.p[{r_rctr}] + {RC_WORDS // 2 * j}, "
                           f"(u64*)&tm_rcnt{j}[threadIdx.x >> 6], {w.el[0]}, tm_rawcap{j})", C.I32, "sl")
             return [t, Val([sl], (), C.I32)]
-        sl = em_.bind(f"(i32)tm_rclaim(&((u64*)P.p[{r_rctr}])[{2 * j}], &tm_rbase{j}[threadIdx.x >> 6], "
-                      f"&tm_rleft{j}[threadIdx.x >> 6], &tm_rcnt{j}[threadIdx.x >> 6], {w.el[0]}, tm_rawcap{j})",
+        sl = em_.bind(f"(i32)tm_rclaim<{rec_info[j]['segments']}, {SHARD_WORDS // 2}>((u64*)P.p[{r_rctr}] + "
+                      f"{RC_WORDS // 2 * j}, &tm_rbase{j}[threadIdx.x >> 6], &tm_rleft{j}[threadIdx.x >> 6], "
+                      f"&tm_rcnt{j}[threadIdx.x >> 6], &tm_rseg{j}[threadIdx.x >> 6], {w.el[0]}, tm_rawseg{j})",
                       C.I32, "sl")
         return [t, Val([sl], (), C.I32)]
     em.hooks["tallymap_claim"] = claim_rule
@@ -1015,7 +1044,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         if k in r_scr:
             zero_words.append((r_scr[k], scratch_words(s)))
     if recs:
-        zero_words.append((r_rctr, 4 * len(recs)))
+        zero_words.append((r_rctr, RC_WORDS * len(recs)))
     zero_words += [(r_ctl, n_ctl), (r_stats, 5)]
     zl = []
     for b, nw in zero_words:
@@ -1042,7 +1071,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     poison = [k for k in outs if prog.tallies[k].dtype in (C.F32, C.F64) and k not in raw]
     bad = ["TM_CTL[2] != 0u"] if prog.trunc is not None else []
     # a Records output past its capacity poisons every float output of the call (reference _api.py:120-131)
-    bad += [f"((const u64*)P.p[{r_rctr}])[{2 * ri['ctr'] + 1}] > {ri['capacity']}ull" for ri in rec_info]
+    bad += [f"((const u64*)P.p[{r_rctr}])[{RC_WORDS // 2 * ri['ctr'] + RC_TOTAL}] > {ri['capacity']}ull"
+            for ri in rec_info]
     if Q is not None:          # a dropped child (tm_qnext counts them from the generations' tickets)
         bad.append("TM_STATS[1] != 0")
     if bad and poison:
@@ -1106,12 +1136,16 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     if Q is not None:          # a later generation (tm_n_arg < 0) takes its item count from tm_qnext's word
         body.append(f"  const i64 n_items = tm_n_arg >= 0 ? tm_n_arg : (i64)(tm_ctr[20] < {Q}ull ? tm_ctr[20] : {Q}ull);")
     for ri in rec_info:        # each wave's Records batch state (tm_rclaim) and the raw buffers' length
-        j, w = ri["ctr"], block // 64
+        j, w, S, cap = ri["ctr"], block // 64, ri["segments"], ri["capacity"]
         body.append(f"  __shared__ u64 tm_rbase{j}[{w}], tm_rcnt{j}[{w}];")
-        body.append(f"  __shared__ u32 tm_rleft{j}[{w}];")
+        body.append(f"  __shared__ u32 tm_rleft{j}[{w}], tm_rseg{j}[{w}];")
         body.append(f"  if ((threadIdx.x & 63u) == 0u) {{ tm_rbase{j}[threadIdx.x >> 6] = 0ull; "
-                    f"tm_rcnt{j}[threadIdx.x >> 6] = 0ull; tm_rleft{j}[threadIdx.x >> 6] = 0u; }}")
-        body.append(f"  const u64 tm_rawcap{j} = {ri['capacity']}ull + (u64)tm_grid * {w}ull * (TM_RB - 1ull);")
+                    f"tm_rcnt{j}[threadIdx.x >> 6] = 0ull; tm_rleft{j}[threadIdx.x >> 6] = 0u; "
+                    f"tm_rseg{j}[threadIdx.x >> 6] = blockIdx.x % {S}u; }}")
+        body.append(f"  const u64 tm_rawseg{j} = " + (
+            f"{cap}ull + (u64)tm_grid * {w * (RB - 1)}ull;" if S == 1 else
+            f"({-(-cap // RB)}ull + (u64)tm_grid * {w}ull + {S - 1}ull) / {S}ull * {RB}ull;"))
+        body.append(f"  const u64 tm_rawcap{j} = tm_rawseg{j} * {S}ull;")
     if Q is not None:          # the spawn ticket counter; each wave's staging rows and their count
         body.append("  u64* const tm_qctr = tm_ctr + 16;")
         if QS:
@@ -1403,16 +1437,18 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         body.append("    }")
         body.append("  }")
     body.append("  if (tm_drop) atomicAdd(&TM_STATS[4], tm_drop);")
-    for ri in rec_info:        # each wave: its records into the exact count, its last batch's unused slots listed
-        j, w, fin = ri["ctr"], block // 64, f"((u64*)P.p[{ri['fin']}])"
-        body.append("  if ((threadIdx.x & 63u) == 0u) {")
-        body.append(f"    const u64 tm_w = (u64)blockIdx.x * {w} + (threadIdx.x >> 6), tm_c = tm_rcnt{j}[threadIdx.x >> 6];")
-        body.append(f"    const u64 tm_b = tm_rbase{j}[threadIdx.x >> 6];")
+    for ri in rec_info:        # each wave: its records into the exact count, its last batch's unused slots keyed 0
+        j, w = ri["ctr"], block // 64
+        rc = f"((u64*)P.p[{r_rctr}] + {RC_WORDS // 2 * j})"
+        body.append("  {")
+        body.append(f"    const u64 tm_c = tm_rcnt{j}[threadIdx.x >> 6], tm_b = tm_rbase{j}[threadIdx.x >> 6];")
         body.append(f"    const u32 tm_l = tm_rleft{j}[threadIdx.x >> 6];")
-        body.append(f"    if (tm_c) atomicAdd(&((u64*)P.p[{r_rctr}])[{2 * j + 1}], tm_c);")
-        body.append(f"    {fin}[1 + 2 * tm_w] = tm_c ? tm_b + (TM_RB - tm_l) : 0ull;")
-        body.append(f"    {fin}[2 + 2 * tm_w] = tm_c ? tm_b + TM_RB : 0ull;")
-        body.append(f"    if (tm_w == 0) {fin}[0] = (u64)tm_grid * {w};")
+        body.append("    for (u32 q = (u32)tm_lane(); q < tm_l; q += 64u) {")
+        body.append("      const u64 s = tm_b + (TM_RB - tm_l) + q;")
+        body.append(f"      if (s < tm_rawcap{j}) ((i32*)P.p[{r_out[ri['ki']]}])[s] = 0;")
+        body.append("    }")
+        body.append(f"    if ((threadIdx.x & 63u) == 0u && tm_c != 0ull) atomicAdd(&{rc}[{RC_TOTAL}], tm_c);")
+        body.append(f"    if (blockIdx.x == 0u && threadIdx.x == 0u) {rc}[{RC_TOTAL + 1}] = (u64)tm_grid * {w}u;")
         body.append("  }")
     body.append("  if (tm_ntr) atomicAdd(&TM_CTL[2], tm_ntr);")
     ldecl = []
@@ -1487,17 +1523,17 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     aux = []
     # any truncation or any Records output past its capacity: every float output NaN, every integer record field -1
     rbad = " || ".join((["TM_CTL[2] != 0u"] if prog.trunc is not None else [])
-                       + [f"((const u64*)P.p[{r_rctr}])[{2 * ri['ctr'] + 1}] > {ri['capacity']}ull"
+                       + [f"((const u64*)P.p[{r_rctr}])[{RC_WORDS // 2 * ri['ctr'] + RC_TOTAL}] > {ri['capacity']}ull"
                           for ri in rec_info])
     for ri in rec_info:
         src.append(_records_passes(ri, r_rctr, r_out, r_ys[ri["count"]], r_rex, r_rbs, prog, rbad))
         j = ri["ctr"]
         cap = ri["capacity"]
-        aux += [(f"tm_rholes{j}", "waves", 256, cap), (f"tm_rscan{j}", "items", 1024, cap),
+        aux += [(f"tm_rscan{j}", "items", 1024, cap),
                 (f"tm_rtop{j}", "one", 1024, cap), (f"tm_rcanon{j}", "cap", 256, cap)]
     L = Layout(n_in=n_in, res=res, n_zero=n_zero, r_out=r_out, r_ctl=r_ctl, r_stats=r_stats, r_ys=r_ys,
                flags=flags, mode=mode, priv=priv, zero_words=zero_words, r_q=r_q,
-               records=[dict(name=ri["name"], capacity=ri["capacity"], r_ctr=(r_rctr, 2 * ri["ctr"] + 1),
+               records=[dict(name=ri["name"], capacity=ri["capacity"], r_ctr=(r_rctr, RC_WORDS // 2 * ri["ctr"] + RC_TOTAL),
                              fields={f: rr for f, (_, rr) in ri["fields"].items()}) for ri in rec_info], aux=aux,
                scratch=sorted(r_scr.values()) + [r_ctl])
     return "\n".join(src) + "\n", L
