@@ -714,8 +714,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         t, w, leaves = ins[0], ins[1], ins[2:]
         if Q is None or len(leaves) != len(qav):
             raise RuntimeError("internal: a spawn in a program without a queue of its per-item operands")
+        when = f"(tm_lead && {w.el[0]})" if lead[0] else w.el[0]
         if not QS or em_.div:
-            tq = em_.bind(f"tm_qclaim(tm_qctr, {w.el[0]})", C.I64, "tq")
+            tq = em_.bind(f"tm_qclaim(tm_qctr, {when})", C.I64, "tq")
             em_.open(f"if ((u64){tq} < {int(Q)}ull)")
             for i, (lv, a) in enumerate(zip(leaves, qav)):
                 ct, n = ctype(a.dtype), max(1, a.size)
@@ -723,7 +724,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                     em_.line(f"(({ct}*)P.p[{r_q[i]}])[{tq} * {n} + {el}] = {lv.el[el]};")
             em_.close()
             return t
-        wv = em_.bind(w.el[0], C.BOOL, "sw")
+        wv = em_.bind(when, C.BOOL, "sw")
         m, nn, q = em_.fresh("sm"), em_.fresh("sn"), em_.fresh("sq")
         em_.line(f"const u64 {m} = tm_ballot({wv});")
         em_.open(f"if ({m} != 0ull)")
@@ -1022,7 +1023,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             return head, em.lines, len(words)
         if compact:
             pl_ahead = Ahead.plan(we, lambda v: isinstance(v, C.Var) and isinstance(env.get(v.id), VTally), cost) \
-                if Q is None and not recs else None
+                if not recs else None
             tail_lines = tail_ahead(pl_ahead) if pl_ahead is not None else step(5, False)
 
     # ------------------------------------------------------------------------------------ assemble
@@ -1135,6 +1136,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("  u64* const tm_ctr = (u64*)P.p[%d];" % r_ctl)
     if Q is not None:          # a later generation (tm_n_arg < 0) takes its item count from tm_qnext's word
         body.append(f"  const i64 n_items = tm_n_arg >= 0 ? tm_n_arg : (i64)(tm_ctr[20] < {Q}ull ? tm_ctr[20] : {Q}ull);")
+        body.append("  if (n_items <= 0) return;                // (a generation queued past the last)")
     for ri in rec_info:        # each wave's Records batch state (tm_rclaim) and the raw buffers' length
         j, w, S, cap = ri["ctr"], block // 64, ri["segments"], ri["capacity"]
         body.append(f"  __shared__ u64 tm_rbase{j}[{w}], tm_rcnt{j}[{w}];")

@@ -95,3 +95,16 @@ def test_taped_gradient_matches_the_plain_loop(n):
         got.append(tm.grad(f, {"hist": w}, argnums=(0, 2))(*args))
     assert torch.equal(got[0][0], got[1][0])
     assert torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 300, 3000])
+def test_spawning_program_matches_the_plain_loop(n):
+    """the shower: the same tree (children spawned once per item, by one lane of its group), the same exact deposits."""
+    import torch
+    p = problems.PROBLEMS["shower"]
+    args = p["inputs"](n)[0]
+    got = [tm.vmap(p["item"], outputs=_exact(p["outputs"]), in_axes=p["in_axes"], spawn=tm.Queue(max(n, 64)), **o)(*args)
+           for o in (dict(), dict(compact=0))]
+    for k in got[0].stats:
+        assert int(got[0].stats[k].item()) == int(got[1].stats[k].item()), k
+    assert torch.equal(got[0].outputs["dep"], got[1].outputs["dep"])
