@@ -601,7 +601,8 @@ def _truncation(trunc, ntr, N):
     if trunc is not None:
         return trunc, ntr
     import torch
-    return torch.zeros((N,), dtype=torch.bool, device="cuda"), torch.zeros((), dtype=torch.int32, device="cuda")
+    z = torch.zeros((1 + (N + 3) // 4,), dtype=torch.int32, device="cuda")        # (one fill for both)
+    return z[1:].view(torch.bool)[:N], z[0]
 
 
 def _record_outputs(prog, o, res_out, stats):
@@ -674,7 +675,35 @@ def vmap(fn=None, *, outputs, in_axes=0, max_steps=None, spawn=None, backend="au
 
     spec_key = tuple(sorted((n, repr(v)) for n, v in outs_spec.items()))     # (the program cache key's outputs)
 
+    calls = {}          # (program kind, per argument: shape, dtype) -> prepare's answer for calls with array arguments
+
     def prepare(args, spawn_mode=None):
+        """(program, meta, per-item operands, broadcast operands, N, axes) of a call."""
+        # a repeated call with arrays alone (no pytrees, no Python scalars) differs from an earlier one in its data
+        # only: shapes and types decide the program
+        key = [spawn_mode]
+        for a in args:
+            sh, dt = getattr(a, "shape", None), getattr(a, "dtype", None)
+            if sh is None or dt is None:
+                key = None
+                break
+            key.append(sh)
+            key.append(dt)
+        if key is not None:
+            key = tuple(key)
+            hit = calls.get(key)
+            if hit is not None:
+                prog, meta, mapped_at, bcast_at, N, axes = hit
+                return prog, meta, [args[i] for i in mapped_at], [args[i] for i in bcast_at], N, axes
+        prog, meta, pi, bc, N, axes = prepare_call(args, spawn_mode)
+        if key is not None:
+            if len(calls) >= PROG_CACHE:
+                calls.clear()
+            calls[key] = (prog, meta, [i for i, x in enumerate(axes) if x == 0],
+                          [i for i, x in enumerate(axes) if x is None], N, axes)
+        return prog, meta, pi, bc, N, axes
+
+    def prepare_call(args, spawn_mode):
         axes = in_axes if isinstance(in_axes, (tuple, list)) else (in_axes,) * len(args)
         if len(axes) != len(args) or any(a not in (0, None) for a in axes):
             raise ValueError("tallymap: in_axes must be 0/None or a tuple of 0/None per positional argument")

@@ -76,6 +76,12 @@ def device_tensor(x, dtype):
     return torch.from_numpy(a).to("cuda")
 
 
+def raw_stream():
+    """torch's current stream on the current device, as a hipStream_t."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def compiled(prog, opts, adjoint=None):
     """the registered kernel of prog under opts (in-memory LRU, then the disk cache, then hipRTC)."""
     block = int(opts.get("block", K.BLOCK))
@@ -169,7 +175,7 @@ def _queue(c, ins, outs, N, n_zero, flags, stream=None, n_main=None):
     L = c.layout
     bufs = [t.data_ptr() for t in ins] + [t.data_ptr() for t in outs]
     arr = (ctypes.c_void_p * len(bufs))(*bufs)
-    s = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+    s = stream if stream is not None else raw_stream()
     Cm.check(Cm.lib().tm_launch(c.id, ctypes.c_void_p(s), arr, len(bufs), n_zero, flags,
                                 N if n_main is None else n_main, c.block))
     if n_main == 0:
@@ -207,7 +213,7 @@ def launch_noalloc(c, ins, N, stream=None):
     arr = (ctypes.c_void_p * len(bufs))(*bufs)
     sl = (ctypes.c_int * max(1, len(slots)))(*slots)
     nb = (ctypes.c_longlong * max(1, len(nbytes)))(*nbytes)
-    s = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+    s = stream if stream is not None else raw_stream()
     Cm.check(Cm.lib().tm_launch_noalloc(c.id, ctypes.c_void_p(s), arr, len(bufs), sl, nb, len(slots), L.n_zero,
                                         L.flags, N, c.block))
     return outs
@@ -343,7 +349,7 @@ def _aux(c, name, bufs, n_items, grid=1, block=64, stream=None):
 
     import torch
     arr = (ctypes.c_void_p * len(bufs))(*[t.data_ptr() for t in bufs])
-    s = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+    s = stream if stream is not None else raw_stream()
     Cm.check(Cm.lib().tm_launch_aux(c.id, name.encode(), ctypes.c_void_p(s), arr, len(bufs), n_items, grid, block))
 
 

@@ -89,6 +89,7 @@ struct Loaded {
   std::map<int, int> occ;       // block size -> blocks per CU of tm_main
   int cap = 0;                  // the module's tm_grid_cap: at most this many blocks per CU (0: the occupancy)
   int spread = 0;               // the module's tm_spread: lanes per item a small launch spreads to (0: one)
+  int priv = 0;                 // private (scratch) bytes per lane of the item loop
   int block0 = 0, occ0 = 0;     // block size and blocks per CU of the first tm_main launch (0: not launched yet)
 };
 
@@ -170,6 +171,10 @@ int loaded(long long id, std::shared_ptr<Loaded>* out) {
       !probe(&L->main, "tm_fused"))
     return fail("tallymap_rocm: %s has no item loop (tm_main, tm_adjoint, tm_count or tm_fused)",
                 pr->second->note.c_str());
+  if (g_rt.hipFuncGetAttribute(&L->priv, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, L->main) != hipSuccess) {
+    L->priv = 0;
+    (void)g_rt.hipGetLastError();
+  }
   probe(&L->zero, "tm_zero");
   probe(&L->post, "tm_post");
   // a module may cap its persistent grid (int tm_grid_cap, blocks per CU) and spread small launches over more lanes
@@ -309,11 +314,9 @@ int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, 
       return fail("tallymap_rocm: flags bit 4 needs a spawning program (program %lld has no tm_qnext)", id);
     karg = -1;
   }
-  int priv = 0;
-  if (g_rt.hipFuncGetAttribute(&priv, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, L->main) != hipSuccess) priv = 0;
-  if (priv > MAX_PRIVATE)
+  if (L->priv > MAX_PRIVATE)
     return fail("tallymap_rocm: program %lld needs %d private bytes per lane (limit %lld): refusing to launch", id,
-                priv, MAX_PRIVATE);
+                L->priv, MAX_PRIVATE);
   int occ = 1;
   if (occupancy(*L, block, &occ)) return 1;
   std::vector<char> args(sizeof(void*) * n + sizeof(long long));
