@@ -844,13 +844,15 @@ def vjp(mapped, *args, argnums=None, n_active=None):
     reverse launch alone (the tape stays allocated while the pullback lives; the option rev_record=False runs the
     plain forward and the whole adjoint at pullback time instead).
     Where the gradient runs as tangent lanes (option grad_mode; by default a few broadcast elements through a loop
-    carry), the forward call is the jvp launch with one lane per differentiated element and the pullback is a
-    contraction of its tangent outputs with the cotangents, on the device, with no launch of its own (plain
-    float32 tallies' tangents accumulate in float64 atomics: reproducible to float64 reassociation; grad_mode=
-    'reverse' gives the replay adjoint's exact, bitwise reproducible broadcast cotangents)."""
+    carry, or, in large calls, where one launch of them costs less than the forward and the adjoint), the forward call
+    is the jvp launch with one lane per differentiated element and the pullback is a contraction of its tangent
+    outputs with the cotangents, on the device, with no launch of its own (plain float32 tallies' tangents accumulate
+    in float64 atomics: reproducible to float64 reassociation; grad_mode='reverse' gives the replay adjoint's exact,
+    bitwise reproducible broadcast cotangents)."""
     m = mapped._sized(args, n_active)
     prog, meta, pi, bc, N, axes = m._prepare(args)
-    tg = _tangent_plan(m, prog, args, axes, argnums)
+    tg = _tangent_plan(m, prog, args, axes, argnums,
+                       pair=(N if n_active is None else int(n_active)) >= LANES_PAIR_ITEMS)
     if tg is not None:
         return _tangent_vjp(m, args, tg, n_active)
     if prog.spawn is None and not prog.records:
@@ -1057,7 +1059,7 @@ _UNITS = {}                    # (shape, dtype, element) -> the unit tangent on 
 _TPLAN = collections.OrderedDict()   # (program, argnums, axes, mode, argument trees) -> _tangent_plan's answer
 
 
-def _tangent_plan(m, prog, args, axes, argnums):
+def _tangent_plan(m, prog, args, axes, argnums, pair=False):
     """how the gradient w.r.t. argnums is computed (option grad_mode): None for the replay adjoint (reverse mode),
     else (spec, wrt, lanes, bav) with lanes = [(broadcast operand, flat element)], one forward-mode tangent lane per
     float32 element of the broadcast arguments (bav: the program's broadcast operand avals).
@@ -1069,7 +1071,9 @@ def _tangent_plan(m, prog, args, axes, argnums):
     they are cheaper: every differentiated argument is broadcast, P <= TANGENT_MAX, and a loop carry needs the
     reverse sweep (the tape adjoint; a forward-only adjoint is one launch already) or the call spawns (the tree
     adjoint is a recording forward, a canonical ordering and a count and a reverse launch per generation; the lanes
-    are one forward through the generations, the children carrying their parents' tangents).  'reverse' always
+    are one forward through the generations, the children carrying their parents' tangents).  pair: the caller needs
+    the forward's outputs before the cotangent (vjp), so a forward-only adjoint is a second launch after the
+    forward's; the lanes are taken where one launch of them costs less (_lanes_beat_pair).  'reverse' always
     replays; 'tangent' takes the lanes whenever the arguments allow (any P, 16 lanes per launch).  Per-item
     arguments and Records outputs always replay."""
     mode = m._opts.get("grad_mode") or "auto"
@@ -1078,17 +1082,48 @@ def _tangent_plan(m, prog, args, axes, argnums):
     if mode == "reverse":
         return None
     an = _argnums(argnums, len(args))
-    key = (prog.digest(), an, tuple(axes), mode, tuple(repr(flatten(args[a])[1]) for a in an))
+    key = (prog.digest(), an, tuple(axes), mode, pair, tuple(repr(flatten(args[a])[1]) for a in an))
     hit = _TPLAN.get(key, _TPLAN)
     if hit is not _TPLAN:
         return hit
-    plan = _TPLAN[key] = _tangent_plan_of(prog, args, axes, an, mode)
+    plan = _TPLAN[key] = _tangent_plan_of(prog, args, axes, an, mode, pair)
     while len(_TPLAN) > PROG_CACHE:
         _TPLAN.popitem(last=False)
     return plan
 
 
-def _tangent_plan_of(prog, args, axes, an, mode):
+LANES_PAIR = 0.75              # vjp takes lanes for a forward-only adjoint when a lane step costs at most this share of a
+                               # forward step and an adjoint step together (kernel.cost): the random walk problem's
+                               # three lanes are 0.60 of them, and its loss gradient at 4,194,304 items took 1,156 us by
+                               # the two launches against 610 by one ...
+LANES_PAIR_ITEMS = 1 << 19     # ... in calls of at least this many items: the contraction with the cotangent is ~60 us of
+                               # small device operations (the same gradient at 1,100,000 items: 422 us against 238, at
+                               # 100,000 126 against 184)
+
+
+def _lanes_beat_pair(prog, wrt, nlanes):
+    """whether one launch of the program with its tangent lanes costs less than the forward launch and the forward-only
+    adjoint's: by the static cost of a step of each (kernel.cost), and only where every float32 output's tangent is
+    held in float64 in LDS (a larger tally's float32 global atomics would cost precision and time)."""
+    from . import backend as B
+    from .backend import kernel as K
+    from .backend import reverse as R
+    from .backend import simplify
+    if K._split(prog.jaxpr) is None:
+        return False
+    q = _jvp_prog(prog, (False,) * prog.nP, tuple(i in wrt[1] for i in range(prog.nB)), nlanes, True)
+    if any(t.kind == "sum" and t.dtype == C.F32 and not t.exact for t in q.tallies[prog.nT:]):
+        return False
+    adj, pl = B._adjoint(prog, wrt)
+
+    def step(p):
+        at = K._split(p.jaxpr)
+        return None if at is None else K.cost(simplify.cse(p.jaxpr.eqns[at].params["body_jaxpr"]).eqns)
+    costs = [step(p) for p in (q, prog, R.forward_only_program(adj, pl))]
+    return None not in costs and costs[0] <= LANES_PAIR * (costs[1] + costs[2])
+
+
+def _tangent_plan_of(prog, args, axes, an, mode, pair):
     why = None
     if prog.records:
         why = "Records outputs are differentiated by the replay adjoint"
@@ -1104,7 +1139,7 @@ def _tangent_plan_of(prog, args, axes, an, mode):
     if why is not None or not lanes or len(lanes) > TANGENT_MAX:
         return None
     from . import backend as B
-    if prog.spawn is None and not B.needs_sweep(prog, wrt):
+    if prog.spawn is None and not B.needs_sweep(prog, wrt) and not (pair and _lanes_beat_pair(prog, wrt, len(lanes))):
         return None
     return spec, wrt, lanes, bav
 

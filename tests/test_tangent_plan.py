@@ -94,3 +94,24 @@ def test_auto_takes_lanes_for_a_spawning_call():
     assert _plan(rcfg, (x, th), 1) is None
     with pytest.raises(tm.UnsupportedError):
         _plan(rcfg, (x, th), 1, grad_mode="tangent")
+
+
+def test_vjp_takes_lanes_where_they_cost_less_than_two_launches():
+    """vjp needs the outputs before the cotangent: forward and forward-only adjoint are two launches, the lanes one.
+    Taken for small float32 sums and few elements; not where a tangent would leave float64 LDS sums (the disk's maps),
+    not with 'reverse', and grad / value_and_grad (one launch by the adjoint) stay."""
+    from tallymap_amd import problems
+
+    def plan(f, args, argnum, pair):
+        m = f._sized(args, None)
+        prog, _, _, _, _, axes = m._prepare(args)
+        return _api._tangent_plan(m, prog, args, axes, argnum, pair=pair)
+    rw = problems.PROBLEMS["random_walk"]
+    args = rw["inputs"](64)[0]
+    p = plan(problems.mapped("random_walk"), args, 2, True)
+    assert p is not None and p[2] == [(0, 0), (0, 1), (0, 2)]
+    assert plan(problems.mapped("random_walk"), args, 2, False) is None
+    assert plan(problems.mapped("random_walk", grad_mode="reverse"), args, 2, True) is None
+    for cfg, inputs, pos in ((configs.c4_config(64), configs.c4_inputs(64), 3), (configs.C1, configs.c1_inputs(64), 0)):
+        f = tm.vmap(cfg["item"], outputs=cfg["outputs"], in_axes=cfg["in_axes"], max_steps=cfg["max_steps"])
+        assert plan(f, inputs, pos, True) is None
