@@ -49,7 +49,8 @@ int tm_register(long long id, const void* image, size_t n, const char* note);
  * tm_qnext after the previous generation), n_items its upper bound (the queue capacity), which sizes the grid.
  * block: threads per block of tm_main (the program's compiled block size).  The grid is persistent:
  * min(ceil(n_items / block), compute units x blocks per CU), blocks per CU being tm_main's occupancy, or the module's
- * `int tm_grid_cap` (a __constant__, read when the module loads) where that is lower.
+ * `int tm_grid_cap` (a __constant__, read when the module loads) where that is lower; with `int tm_spread` above 1, a
+ * launch of fewer items than those lanes takes up to tm_spread lanes per item (idle lanes compute draws ahead).
  * Asynchronous: nothing waits for the kernels. */
 int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, int flags, long long n_items,
               int block);
@@ -83,8 +84,8 @@ void tm_free(void* p);
 int tallymap_register(int64_t id, const char* data, size_t n, const char* note);
 int tallymap_kernel_info(int64_t id, long long* out);
 
-/* Bytes of the device array tm_launch_noalloc places scratch buffers in: one per GPU the library runs on, held
- * until the process ends. */
+/* Bytes of the device array tm_launch_noalloc places scratch buffers in (and 16,608 more for the claim counters of a
+ * program's item ranges): one per GPU the library runs on, held until the process ends. */
 #define TM_NOALLOC_SCRATCH_BYTES (32u << 20)
 
 /* tm_launch for callers that cannot allocate device memory -- code under HIP graph capture, tight serving loops,

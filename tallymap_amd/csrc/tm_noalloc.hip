@@ -17,7 +17,11 @@
 
 int tm_fail_msg(const char* msg);     // tm_shim.cc: sets tm_last_error(), returns 1
 
-static __device__ __align__(256) unsigned char scratch[TM_NOALLOC_SCRATCH_BYTES];
+// Beside TM_NOALLOC_SCRATCH_BYTES, room for the claim counters of a program's item ranges: its control words are 4,160
+// u32, 16,608 bytes more than the 8 they took with one counter, and a program whose scratch then filled the array
+// still fits.
+static constexpr unsigned long long kClaimBytes = (4160 - 8) * 4;
+static __device__ __align__(256) unsigned char scratch[TM_NOALLOC_SCRATCH_BYTES + kClaimBytes];
 
 namespace {
 
@@ -88,7 +92,8 @@ extern "C" int tm_launch_noalloc(long long id, void* stream, void* const* bufs, 
     seen[s] = true;
     const unsigned long long at = (end + kAlign - 1) / kAlign * kAlign;
     const unsigned long long b = static_cast<unsigned long long>(bytes[j]);
-    if (at > TM_NOALLOC_SCRATCH_BYTES || b > TM_NOALLOC_SCRATCH_BYTES - at)
+    if (b > TM_NOALLOC_SCRATCH_BYTES || at > TM_NOALLOC_SCRATCH_BYTES + kClaimBytes ||
+        b > TM_NOALLOC_SCRATCH_BYTES + kClaimBytes - at)
       return err("tallymap_rocm: tm_launch_noalloc: the program's scratch needs more than the %u bytes of the "
                  "no-alloc array (slot %d: %lld bytes at offset %llu); use tm_launch with caller buffers",
                  TM_NOALLOC_SCRATCH_BYTES, s, bytes[j], at);
