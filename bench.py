@@ -57,15 +57,15 @@ def _classes(*counts):
     return {"SQ_INSTS_VALU_" + c: float(n) for c, n in zip(VALU_CLASSES, counts)}
 
 
-MEASURED = {"fused": {"code": "869dad0bad514189", "traffic": 76_871_377, "valu_insts": 6.6894e+09,
-                       "valu_classes": _classes(1.833e+09, 6.588e+07, 1.432e+08, 8.591e+07, 0, 0,
-                                                1.77e+08, 1.249e+08, 5.644e+08, 5.176e+06, 1.432e+08)},
-            "forward": {"code": "646dbd1780dfad7f", "traffic": 77_564_904, "valu_insts": 6.6871e+09,
-                        "valu_classes": _classes(1.832e+09, 6.586e+07, 1.431e+08, 8.588e+07, 0, 0,
-                                                 1.77e+08, 1.249e+08, 5.644e+08, 5.176e+06, 1.431e+08)},
-            "gradient": {"code": "2c3a66dcd7cd746b", "traffic": 56_478_890, "valu_insts": 6.3393e+09,
-                         "valu_classes": _classes(1.772e+09, 6.203e+07, 1.435e+08, 5.741e+07, 0, 0,
-                                                  1.774e+08, 1.252e+08, 5.657e+08, 5.176e+06, 1.148e+08)}}
+MEASURED = {"fused": {"code": "fecd2447bd79fc61", "traffic": 82_477_514, "valu_insts": 6.1971e+09,
+                       "valu_classes": _classes(1.836e+09, 4.837e+07, 1.405e+08, 8.641e+07, 0, 0,
+                                                1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
+            "forward": {"code": "a7ef3cc5a67dd356", "traffic": 83_846_204, "valu_insts": 6.1290e+09,
+                        "valu_classes": _classes(1.836e+09, 4.838e+07, 1.404e+08, 8.639e+07, 0, 0,
+                                                 1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
+            "gradient": {"code": "47f260042cd43e9e", "traffic": 62_372_947, "valu_insts": 5.8874e+09,
+                         "valu_classes": _classes(1.739e+09, 4.388e+07, 1.406e+08, 5.411e+07, 0, 0,
+                                                  1.675e+08, 1.186e+08, 5.375e+08, 5.173e+06, 1.082e+08)}}
 
 
 def code_keys(f, dev):
@@ -115,7 +115,7 @@ def measured(kind, field, key, n):
 
 def valu_roofline(kind, key, n, ms):
     """the resource that binds C2's kernels: VALU issue (the HBM roofline is the contract's; the kernel reads 17 B
-    and runs ~406 steps of ~230 VALU instructions per item).  peak: the fastest VALU issue rate measured live on this
+    and runs ~405 steps of ~210 VALU instructions per item).  peak: the fastest VALU issue rate measured live on this
     GPU (backend/valu.py: 32-bit integer and fp32 add / mul, xor), every pattern's rate beside it; achieved: the
     launch's SQ_INSTS_VALU over its duration.  issue_bound_ms: the shortest time the chip can issue that launch's
     instructions in, each SQ_INSTS_VALU_<class> count over the fastest measured rate of the instructions that class
@@ -702,8 +702,8 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "algorithmic_bytes_per_launch": bpi * N,
-                     "binding_resource": "VALU issue, not HBM: the kernel moves 17 B per item and runs ~406 "
-                                         "steps of ~230 VALU instructions per item; its bound and fraction are "
+                     "binding_resource": "VALU issue, not HBM: the kernel moves 17 B per item and runs ~405 "
+                                         "steps of ~210 VALU instructions per item; its bound and fraction are "
                                          "valu_roofline's"},
         "valu_roofline": valu_roofline(dom, ckeys[dom], N, dom_ms) if not a.no_valu_rates else None,
     }

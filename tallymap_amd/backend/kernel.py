@@ -11,10 +11,11 @@ The first group of results (up to stats) is zeroed by tm_zero before tm_main run
 tm_main is the hand-written CDNA4 loop (reference kernel.py:812-838 is the CUDA one it replaces):
   * a persistent grid (256 CUs x achieved occupancy), block BLOCK = 256 (4 wave64s);
   * step-granular refill (the reference's schedule='step', kernel.py:239-295, 469-563): each loop iteration, the
-    lanes of a wave whose item has finished are counted with one ballot, and the wave claims that many
-    consecutive items with ONE atomic (mbcnt gives each idle lane its rank); a lane then runs its item's `pre`,
-    and every live lane runs one (cond, body) step or, when the predicate fails, `post` and writes its per-item
-    results.  A lane never waits for its wave's longest item;
+    lanes of a wave whose item has finished are counted with one ballot and take the next items of the chunk the
+    wave holds (mbcnt gives each idle lane its rank); a chunk is claimed with one atomic on the counter of an item
+    range, of which there are 64.  A lane then runs its item's `pre`, and every live lane runs one (cond, body)
+    step or, when the predicate fails, `post` and writes its per-item results.  A lane never waits for its wave's
+    longest item; lanes left without an item compute the draws of other lanes' coming steps (backend/ahead.py);
   * small tallies privatised in LDS (up to LDS_BYTES per block), flushed once at exit with device atomics;
     larger ones take the global atomic directly;
   * dropped emits and truncations counted in registers, one atomic per lane at exit.
