@@ -10,7 +10,9 @@ and a share of the rest, where it took the whole chain.
 
 `plan` splits the step's equations:
   inv     from loop constants alone: emitted on both sides (the compiler takes them out of the loops)
-  ahead   from counters and loop constants by pure primitives
+  ahead   from counters and loop constants by pure primitives, and by loops whose trip count is a literal: the ahead
+          side also runs for steps past the item's last, and a loop that ends for every counter the item reaches need
+          not end for those
   cheap   the ahead equations of a couple of instructions whose operands the update has anyway (a counter's own
           increment): recomputed there
   update  the rest
@@ -40,6 +42,13 @@ def pure(e):
     if e.prim in ("while", "cond"):
         return all(pure(x) for j in C.subjaxprs(e) for x in j.eqns)
     return e.prim in PURE or (not C.subjaxprs(e) and not e.prim.startswith("tallymap_"))
+
+
+def bounded(e):
+    """whether e ends whatever its operands: every loop in it has a literal trip count."""
+    if e.prim == "while" and not e.params.get("static", False):
+        return False
+    return all(bounded(x) for j in C.subjaxprs(e) for x in j.eqns)
 
 
 def _counters(bj, nb):
@@ -77,7 +86,7 @@ def plan(we, is_tally, cost):
     ahead, update = [], []
     for e in bj.eqns:
         ks = {kind[v.id] for v in e.invars if isinstance(v, C.Var)}
-        if "update" in ks or not pure(e):
+        if "update" in ks or not pure(e) or not bounded(e):
             k = "update"
         elif ks <= {"inv"}:
             k = "inv"

@@ -1000,9 +1000,17 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             head = em.lines
             em.lines, em.ind = [], 4
             lead[0] = True
-            # (the condition on every lane, an item's end under a wave-uniform branch: one lane mask per update)
-            pr = em.run(we.params["cond_jaxpr"], [sval(v) for v in cc_v] + cars)[0]
-            em.line(f"const bool tm_go_on = tm_live && {pr.el[0]};")
+            # (a straight-line condition on every lane, an item's end under a wave-uniform branch: one lane mask per
+            # update.  One with a loop or a branch in it on live lanes alone: the others' state is unset)
+            cj = we.params["cond_jaxpr"]
+            if any(C.subjaxprs(q) for q in cj.eqns):
+                em.line("bool tm_go_on = false;")
+                em.open("if (tm_live)")
+                em.line(f"tm_go_on = {em.run(cj, [sval(v) for v in cc_v] + cars)[0].el[0]};")
+                em.close()
+            else:
+                pr = em.run(cj, [sval(v) for v in cc_v] + cars)[0]
+                em.line(f"const bool tm_go_on = tm_live && {pr.el[0]};")
             em.open("if (tm_ballot(tm_live && !tm_go_on) != 0ull)")
             em.open("if (tm_live && !tm_go_on && tm_lead)")
             lead[0] = False

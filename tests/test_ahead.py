@@ -11,10 +11,14 @@ from tallymap_amd.backend import ahead as A
 from tallymap_amd.backend import kernel as K
 
 
-def _plan(item, outputs, axes, args, max_steps=None):
+def _prog(item, outputs, axes, args, max_steps=None):
     pav = [C.AVal(np.shape(a)[1:], np.asarray(a).dtype) for a, x in zip(args, axes) if x == 0]
     bav = [C.AVal(np.shape(a), np.asarray(a).dtype) for a, x in zip(args, axes) if x is None]
-    prog, _ = build_program(item, outputs, axes, pav, bav, max_steps)
+    return build_program(item, outputs, axes, pav, bav, max_steps)[0]
+
+
+def _plan(item, outputs, axes, args, max_steps=None):
+    prog = _prog(item, outputs, axes, args, max_steps)
     we = prog.jaxpr.eqns[K._split(prog.jaxpr)]
     tallies = {v.id for v in prog.jaxpr.invars[:prog.nT]}
     for e in prog.jaxpr.eqns:           # (a tally stays one through emits)
@@ -35,7 +39,7 @@ def _sound(pl, we):
     same = {v.id for v, o in zip(bj.invars[nb:], bj.outvars) if isinstance(o, C.Var) and o.id == v.id}
     have = {v.id for v in bj.invars[:nb]} | same | {bj.invars[nb + j].id for j in pl.counters}
     for e in pl.ahead:
-        assert A.pure(e)
+        assert A.pure(e) and A.bounded(e)
         assert all(v.id in have for v in e.invars if isinstance(v, C.Var)), e
         have |= {o.id for o in e.outvars}
     assert {id(e) for e in pl.ahead} | {id(e) for e in pl.update} == {id(e) for e in bj.eqns}
@@ -82,3 +86,85 @@ def test_what_counts_as_a_counter():
     assert _walk(lambda key, k, x, m: (u(random.fold_in(key, m)), m + k))[0] is None
     assert _walk(lambda key, k, x, m: (u(random.fold_in(key, m)), m * 2))[0] is None
     assert _walk(lambda key, k, x, m: (u(random.fold_in(key, (x * 100).astype(jnp.int32))), m + 1))[0] is None
+
+
+def _walk_args(n):
+    return np.linspace(0.2, 1.0, n).astype(np.float32), random.split(random.PRNGKey(3), n)
+
+
+# Steps with a loop of their own.  Every loop ends for the counters 0 .. 19 that an item reaches; `up`, `shift` and
+# `branch` never do (or after 2^32 trips) for 21 and on, `levels` doubles its trips with every step.
+def _inner(name, k, u):
+    if name == "up":
+        return lax.while_loop(lambda c: c[0] != 20 - k, lambda c: (c[0] + 1, c[1] * 0.75 + u), (np.int32(0), u))[1]
+    if name == "shift":
+        return lax.while_loop(lambda c: c[0] != 0, lambda c: (c[0] >> 1, c[1] * 0.75 + u), (20 - k, u))[1]
+    if name == "branch":
+        return lax.cond(k % 2 == 0, lambda: _inner("up", k, u), lambda: u)
+    if name == "levels":
+        return lax.fori_loop(0, (0 * k + 1) << k, lambda i, s: s * 0.75 + u, u)
+    assert name == "literal"
+    return lax.fori_loop(0, 100, lambda i, s: s * 0.75 + u, u)
+
+
+def loop_item(name, steps=20):
+    """`steps` steps, each with the loop `name` on the counter and a draw."""
+    def item(t, x, key):
+        def body(c):
+            k, x, t = c
+            u = random.uniform(random.fold_in(key, k))
+            v = _inner(name, k, u)
+            return k + 1, x * (0.5 + 0.125 * u) + v, t.add("h", k % 4, np.int32(1))
+        k, x, t = lax.while_loop(lambda c: c[0] < steps, body, (np.int32(0), x, t))
+        return t, (k, x)
+    return item
+
+
+def condition_item(t, x, key):
+    """a loop condition with a loop in it, which ends for the item's own x > 0 alone."""
+    def cond(c):
+        k, x, t = c
+        n = lax.while_loop(lambda c: c[1] < 1.0, lambda c: (c[0] + 1, c[1] * 2.0), (np.int32(0), x))[0]
+        return n < 12
+
+    def body(c):
+        k, x, t = c
+        u = random.uniform(random.fold_in(key, k))
+        return k + 1, x * (0.5 + 0.5 * u), t.add("h", k % 4, np.int32(1))
+    k, x, t = lax.while_loop(cond, body, (np.int32(0), x, t))
+    return t, (k, x)
+
+
+LOOPS = {"up": 20, "shift": 20, "branch": 20, "levels": 12, "literal": 20}
+
+
+def _ahead_sides(item):
+    """(the plan, the emitted ahead side, the emitted condition) of an item of _walk_args."""
+    spec = ({"h": Sum((4,), dtype=np.int32)}, (0, 0), _walk_args(2))
+    pl, we = _plan(item, *spec)
+    if pl is None:
+        return None, None, None
+    _sound(pl, we)
+    src = K.build(_prog(item, *spec))[0]
+    head = src[src.index("u32 tm_h0 = 0u;"):src.index("u32 tm_n0 = (u32)__builtin_amdgcn_ds_bpermute")]
+    at = src.index("tm_n0 = (u32)__builtin_amdgcn_ds_bpermute(tm_ba + ")
+    return pl, head, src[at:src.index("if (tm_ballot(tm_live && !tm_go_on)", at)]
+
+
+@pytest.mark.parametrize("name", LOOPS)
+def test_loops_without_a_literal_trip_count_stay_in_the_step(name):
+    """the draw is computed ahead, a loop on its counter is not: steps past the item's last have no bound on it."""
+    pl, head, _ = _ahead_sides(loop_item(name, LOOPS[name]))
+    assert pl is not None and "tm_threefry" in head
+    inner = [e for e in pl.ahead if e.prim in ("while", "cond")]
+    if name == "literal":
+        assert len(inner) == 1 and "while (true)" in head
+    else:
+        assert not inner and "while (true)" not in head and any(e.prim in ("while", "cond") for e in pl.update)
+
+
+def test_a_condition_with_a_loop_runs_on_live_lanes_alone():
+    _, _, cond = _ahead_sides(condition_item)
+    assert cond.index("if (tm_live) {") < cond.index("while (true)")
+    _, _, cond = _ahead_sides(loop_item("literal"))
+    assert "if (tm_live)" not in cond

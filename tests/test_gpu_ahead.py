@@ -8,6 +8,8 @@ import tallymap_amd as tm
 from tallymap_amd import configs, lax, problems, random
 from tallymap_amd import numpy as jnp
 
+import test_ahead
+
 pytestmark = pytest.mark.gpu
 # from one item (64 lanes) over the group sizes' edges to more items than a workgroup and than 2 workgroups per CU
 SIZES = (1, 3, 4, 5, 16, 17, 64, 65, 129, 255, 257, 1000, 4099, 131_073)
@@ -108,3 +110,42 @@ def test_spawning_program_matches_the_plain_loop(n):
     for k in got[0].stats:
         assert int(got[0].stats[k].item()) == int(got[1].stats[k].item()), k
     assert torch.equal(got[0].outputs["dep"], got[1].outputs["dep"])
+
+
+def _host_steps(oracle, name, steps, x, keys):
+    """test_ahead's items in numpy float32, step by step -> (steps, the final x) of each item."""
+    f = np.float32
+    out = []
+    for i, x in enumerate(x):
+        k, x = 0, f(x)
+        while (k < steps) if name != "condition" else (np.ceil(-np.log2(x)) < 12):
+            u = f(oracle.uniform(oracle.fold_in(keys[i], k)))
+            if name == "condition":
+                x = x * (f(0.5) + f(0.5) * u)
+            else:
+                trips = {"up": 20 - k, "shift": (20 - k).bit_length(), "branch": 0 if k % 2 else 20 - k,
+                         "levels": 1 << k, "literal": 100}[name]
+                v = u
+                for _ in range(trips):
+                    v = v * f(0.75) + u
+                x = x * (f(0.5) + f(0.125) * u) + v
+            k += 1
+        out.append((k, x))
+    return np.array([k for k, _ in out], np.int32), np.array([x for _, x in out], np.float32)
+
+
+@pytest.mark.parametrize("name", list(test_ahead.LOOPS) + ["condition"])
+def test_steps_with_loops_of_their_own(oracle, name):
+    """loops that end for the steps an item takes and not for those after its last: the plain loop's results, and the
+    host's for the first items."""
+    steps = test_ahead.LOOPS.get(name)
+    item = test_ahead.condition_item if name == "condition" else test_ahead.loop_item(name, steps)
+    for n in (1, 6, 70, 700):
+        print("case:", name, n, flush=True)
+        _pair(lambda o: tm.vmap(item, outputs={"h": tm.Sum((4,), dtype=np.int32)}, in_axes=(0, 0), **o),
+              test_ahead._walk_args, n)
+    x, keys = test_ahead._walk_args(6)
+    r = tm.vmap(item, outputs={"h": tm.Sum((4,), dtype=np.int32)}, in_axes=(0, 0))(x, keys)
+    k, y = _host_steps(oracle, name, steps, x, keys)
+    assert np.array_equal(r.per_item[0].cpu().numpy(), k)
+    assert np.array_equal(r.per_item[1].cpu().numpy(), y)
