@@ -22,6 +22,7 @@ tm_main is the hand-written CDNA4 loop (reference kernel.py:812-838 is the CUDA 
 Programs without exactly one top-level while loop run the item schedule (a lane runs its whole item per claim).
 """
 import dataclasses
+import re
 
 import numpy as np
 
@@ -39,11 +40,14 @@ LDS_F64 = 8192             # of those, float32 sums held as float64 in LDS take 
                            # conflicts), and a float32 value or a sum of them is never a float64 subnormal, so the
                            # compare-and-swap path of tm_ladd_f32 goes too.  Larger tallies keep float32: at 8 bytes a
                            # 4,096-bin map takes a workgroup per CU from the loop, and there the adds are not the bound
+LDS_MAX = 160 << 10        # bytes of LDS a workgroup may have (gfx950)
 LDS_COPIES = 256           # a float64 or count bin of a tally of S bins has up to 16 copies in LDS, S x copies at most
                            # this (8-byte words); a lane adds to copy lane % copies and the flush sums them.  Lanes of
                            # a wave that add to one address take turns: ds_add_f64 cycles per wave64 add and CU (the
                            # probe above, ~18 of them address arithmetic) 392 onto one bin, 111 onto 2, 45 onto 8, 31
-                           # onto 16, 24 onto 64; with 16 copies 18-19 onto 1, 8 or 16 bins, with 4 copies 21 onto 64
+                           # onto 16, 24 onto 64; with 16 copies 18-19 onto 1, 8 or 16 bins, with 4 copies 21 onto 64.
+                           # All copies of a program together take at most LDS_F64 bytes: an unrolled loop over a
+                           # table of 84 weights is 84 counters of 16 bins, 11 KB at one copy and 170 at 16
 REG_BINS = 2               # privatised tallies of at most this many bins accumulate in each lane's registers
 XW = 9                     # int64 words per exact bin (tm_device.h TM_XW: weights 2^(32 j))
 CHUNK = 64
@@ -347,6 +351,18 @@ def _repack_code(decls, cap):
     return pack, unpack, w
 
 
+def lds_bytes(src):
+    """the bytes of the __shared__ arrays and scalars that `src` declares (one declaration a line)."""
+    size = {"double": 8, "float": 4, "bool": 1}
+    n = 0
+    for ct, names in re.findall(r"__shared__ (\w+) ([^;]*);", src):
+        b = size.get(ct) or int(ct[1:]) // 8
+        for nm in names.split(","):
+            m = re.search(r"\[(\d+)\]", nm)
+            n += b * (int(m.group(1)) if m else 1)
+    return n
+
+
 def tally_lds_bytes(s):
     """the LDS bytes a privatised copy of tally spec s takes (exact: XW int64 words per bin; fixed point: an int64
     word, an int32 carry word; else the dtype's size): the kernel privatises tallies in slot order while their
@@ -355,7 +371,7 @@ def tally_lds_bytes(s):
 
 
 def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COMPACT, min_blocks=0,
-          post_batch=POST_BATCH, lds_tables=LDS_TABLES, grid_cap=0):
+          post_batch=POST_BATCH, lds_tables=LDS_TABLES, grid_cap=0, lean=False):
     """-> (HIP source, Layout) of prog's module.  chunk: items a wave claims with one atomic (their per-item operands
     are staged in LDS by one coalesced load, and idle lanes take them from there at step granularity).  compact:
     once every wave of a workgroup has drained the item queue, the waves meet every `compact` iterations and
@@ -374,7 +390,11 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     grid_cap: at most this many workgroups per CU in the item loop's persistent grid (the module's tm_grid_cap,
     which the launcher reads when it loads the module and takes as the occupancy when lower); 0: the occupancy.
     Fewer resident waves give each lane more items (a shorter tail) and a spawning loop's waves fewer concurrent
-    claims and queue flushes, at the cost of latency hiding."""
+    claims and queue flushes, at the cost of latency hiding.
+    lean: no copies of LDS bins and no float64 ones: what a program whose LDS would pass LDS_MAX with them is built
+    as."""
+    opts = dict(block=block, schedule=schedule, refill=refill, chunk=chunk, compact=compact, min_blocks=min_blocks,
+                post_batch=post_batch, lds_tables=lds_tables, grid_cap=grid_cap)
     chunk = max(1, int(chunk))
     compact = max(0, int(compact))
     jx = simplify.drop_draw_clamp(prog.jaxpr)
@@ -467,7 +487,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     # would take 2 x XW registers per bin in every lane -- measured slower on C5's reverse launch -- so it stays in
     # LDS.)
     # float32 sums accumulated as float64 in LDS (LDS_F64), rounded once per workgroup by the flush
-    d64, left = set(), LDS_F64
+    d64, left = set(), 0 if lean else LDS_F64
     for k in priv:
         s = prog.tallies[k]
         if s.dtype == C.F32 and not s.exact and not s.fixed and 8 * s.S <= left:
@@ -480,12 +500,12 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         while R > 1 and (S * R > LDS_COPIES or S * R > words):
             R //= 2
         return R
-    ncopy, words = {}, LDS_F64 // 8
+    ncopy, room = {}, 0 if lean else LDS_F64 // 8
     for k in priv:
         s = prog.tallies[k]
         if k in d64 or (s.dtype == C.F64 and not s.fixed):
-            ncopy[k] = copies(s.S, words)
-            words -= s.S * ncopy[k] if ncopy[k] > 1 else 0
+            ncopy[k] = copies(s.S, room)
+            room -= s.S * ncopy[k] if ncopy[k] > 1 else 0
 
     def copy_of(ei, R):
         """the index of bin ei's copy for this lane."""
@@ -545,7 +565,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             key = (k, int(c.view(np.uint32)))
             if key not in counts:
                 counts[key] = (f"tm_cn{k}_{len(counts)}", c)
-            em_.line(f"atomicAdd(&{counts[key][0]}[{copy_of(ei, copies(s.S, LDS_F64))}], 1ull);")
+            em_.line(f"atomicAdd(&{counts[key][0]}[TM_CN{k}({ei})], 1ull);")
             em_.close()
             return t
         if s.exact:
@@ -1481,8 +1501,15 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             counts[key] = (f"tm_cn{k}_{len(counts)}", c)
         for b, nm in enumerate(names):
             ldecl.append(f"  u32 {nm} = 0u;")
-            body.append(f"  if ({nm} != 0u) atomicAdd(&{counts[key][0]}[{copy_of(b, copies(prog.tallies[k].S, LDS_F64))}], (u64){nm});")
+            body.append(f"  if ({nm} != 0u) atomicAdd(&{counts[key][0]}[TM_CN{k}({b})], (u64){nm});")
     body[body.index("//TM_LANE_DECLS")] = "\n".join(ldecl)
+    # the constants' counters share the copies' words with the sums: every constant of a tally has the same number
+    ccopy = {}
+    for k in sorted({k for k, _ in counts}):
+        S, n = prog.tallies[k].S, sum(kk == k for kk, _ in counts)
+        ccopy[k] = copies(S, room // n)
+        room -= S * n * ccopy[k] if ccopy[k] > 1 else 0
+        src.append(f"#define TM_CN{k}(e) ({copy_of('(e)', ccopy[k])})")
     if priv:
         body.append("  __syncthreads();")
         for k in priv:
@@ -1515,7 +1542,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                             f"if (x != 0.0f) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], x); }}")
                 for (kk, _), (nm, c) in counts.items():
                     if kk == k:
-                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const u64 n = {sum_copies(nm, copies(s.S, LDS_F64))}; "
+                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const u64 n = {sum_copies(nm, ccopy[k])}; "
                                     f"if (n != 0ull) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], "
                                     f"tm_u64_f32(n) * {lit(c, np.float32)}); }}")
             else:
@@ -1525,11 +1552,12 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("}")
     cdecl = []
     for (k, _), (nm, c) in counts.items():
-        S = prog.tallies[k].S
-        S *= copies(S, LDS_F64)
+        S = prog.tallies[k].S * ccopy[k]
         cdecl.append(f"  __shared__ u64 {nm}[{S}];")
         cdecl.append(f"  for (int i = threadIdx.x; i < {S}; i += TM_BLOCK) {nm}[i] = 0ull;")
     body[body.index("//TM_COUNT_DECLS")] = "\n".join(cdecl)
+    if not lean and lds_bytes("\n".join(body)) > LDS_MAX:
+        return build(prog, **opts, lean=True)
     src.append("\n".join(body))
     aux = []
     # any truncation or any Records output past its capacity: every float output NaN, every integer record field -1

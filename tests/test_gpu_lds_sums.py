@@ -51,3 +51,17 @@ def test_non_finite_values_reach_their_bin_only():
     v[0], v[1], v[2], v[6] = np.nan, np.inf, np.inf, -np.inf
     got, _, _ = _run(b, v, 4, np.float32)
     assert np.isnan(got[0]) and got[1] == np.inf and np.isnan(got[2]) and got[3] == 8.0
+
+
+@pytest.mark.parametrize("S, n", [(2, 40), (16, 1), (16, 3), (16, 40), (16, 84), (1024, 19)])
+def test_sums_of_many_constants(S, n):
+    """a counter per constant in LDS: copies of it while the budget lasts, one above, and (1,024 bins of 19 constants)
+    no float64 bins beside them.  Multiples of 1/128 below 2^17: every sum is exact in float32."""
+    def item(t, b):
+        for j in range(n):
+            t = t.add("h", (b + 7 * j) % S, np.float32(1.0 + j / 128.0))
+        return t
+    b = np.random.default_rng(S + n).integers(0, S, 1000).astype(np.int32)
+    want = sum(np.bincount((b + 7 * j) % S, minlength=S) * (1.0 + j / 128.0) for j in range(n))
+    got = tm.vmap(item, outputs={"h": tm.Sum((S,))}, in_axes=(0,))(b).outputs["h"].cpu().numpy()
+    assert np.array_equal(got, want.astype(np.float32))
