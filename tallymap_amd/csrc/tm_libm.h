@@ -359,7 +359,8 @@ TM_FN float tm_sc_poly(double x, double x2, int n, bool flip) {
 // |x| < 120: n = round(x 2/pi) (through 2^24-scaled integer arithmetic), x - n pi/2 with one fma
 TM_FN double tm_sc_reduce_fast(double x, int* np) {
   const double r = x * TM_SC_HPI_INV;
-  const int n = (tm_d2i32(r) + 0x800000) >> 24;    // (any x may come here; the caller replaces what |x| >= 120 gives)
+  // (any x may come here: the add wraps, and the caller replaces what |x| >= 120 gives)
+  const int n = (i32)((u32)tm_d2i32(r) + 0x800000u) >> 24;
   *np = n;
   return __builtin_fma(-(double)n, TM_SC_HPI, x);
 }
