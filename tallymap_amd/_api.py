@@ -684,7 +684,8 @@ def vmap(fn=None, *, outputs, in_axes=0, max_steps=None, spawn=None, backend="au
         key = [spawn_mode]
         for a in args:
             sh, dt = getattr(a, "shape", None), getattr(a, "dtype", None)
-            if sh is None or dt is None:
+            # (a shape of another type may not be hashable; a container of leaves may have fields of these names)
+            if not isinstance(sh, tuple) or dt is None or isinstance(a, (tuple, list, dict)):
                 key = None
                 break
             key.append(sh)

@@ -550,3 +550,29 @@ def test_transcendentals_lower_to_the_glibc_restatements(dt):
     glibc_bitwise = {n for n in unary + binary if G.LIBM[(n, t)].startswith("tm_")}
     rest = {"cbrt"} if dt == np.float32 else {"sin", "cos", "tan", "asin", "acos", "atan", "atan2", "cbrt"}
     assert set(unary + binary) - glibc_bitwise == rest
+
+
+class _Listed:
+    """an array whose shape is a list, as some array libraries give it."""
+    def __init__(self, a):
+        self.a, self.shape, self.dtype = a, list(a.shape), a.dtype
+
+
+class _Grid(dict):
+    """a container of operands with attributes that an array has too."""
+    shape, dtype = (4,), np.dtype(np.float32)
+
+
+def test_a_repeated_call_is_found_by_arrays_alone():
+    """a call's program is looked up by its arguments' shapes and types; an argument whose shape cannot be a key, or a
+    container that has attributes of these names, is described in full each time."""
+    x = np.ones(4, np.float32)
+    f = tm.vmap(lambda t, x: t.add("h", 0, x), outputs={"h": tm.Sum((1,))})
+    p = f._prepare((x,))[0]
+    assert f._prepare((x + 1,))[0] is p and f._prepare((_Listed(x),))[0] is p and f._prepare((_Listed(x),))[4] == 4
+    g = tm.vmap(lambda t, x: t.add("h", 0, x["a"]), outputs={"h": tm.Sum((1,))})
+    for n in (4, 6, 4):
+        got = g._prepare((_Grid(a=np.ones(n, np.float32)),))
+        assert got[4] == n and got[2][0].shape == (n,)
+    for dt in (np.float32, np.int32):
+        assert g._prepare((_Grid(a=np.ones(4, dt)),))[0].p_avals()[0].dtype == dt
