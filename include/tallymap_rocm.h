@@ -46,11 +46,13 @@ int tm_register(long long id, const void* image, size_t n, const char* note);
  * first (it clears the program's accumulators and counters); flags bit 1: run tm_post after tm_main (exact
  * readout, truncation poison); flags bit 2 (value 4, spawning programs only, without tm_zero and tm_post): a later
  * generation of a spawn tree, whose item count tm_main reads from the program's control words (written by
- * tm_qnext after the previous generation), n_items its upper bound (the queue capacity), which sizes the grid.
+ * tm_qnext after the previous generation), n_items its upper bound (the queue capacity), which sizes the grid;
+ * flags bit 3 (value 8): run tm_post after tm_main where the launch spread (below), or with n_items 0 (its float64
+ * sums of small launches then hold what tm_main left; a launch that did not spread has added to the outputs itself).
  * block: threads per block of tm_main (the program's compiled block size).  The grid is persistent:
  * min(ceil(n_items / block), compute units x blocks per CU), blocks per CU being tm_main's occupancy, or the module's
  * `int tm_grid_cap` (a __constant__, read when the module loads) where that is lower; with `int tm_spread` above 1, a
- * launch of fewer items than those lanes takes up to tm_spread lanes per item (idle lanes compute draws ahead).
+ * launch of fewer items than those lanes spreads: up to tm_spread lanes per item (idle lanes compute draws ahead).
  * Asynchronous: nothing waits for the kernels. */
 int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, int flags, long long n_items,
               int block);

@@ -500,7 +500,7 @@ def _records_spawn(prepare, opts, names, args):
     stats = {n: o.stats[ST[n]] for n in ("fixed_point_overflow", "dropped_emits")}
     stats.update((n, o.stats[ST[n]]) for n in ("spawned", "children_dropped", "children_truncated"))
     ys, trunc = _split_ys(prog, list(o.ys))
-    trunc, stats["n_truncated"] = _truncation(trunc, o.n_truncated, N)
+    trunc, stats["n_truncated"] = _truncation(trunc, o, N)
     recs = list(prepare(args)[0].records)      # (name, capacity, fields) of each Records output
     bad, over, offs = _tree_records(o, recs, prog, stats)
     rt = {}
@@ -574,7 +574,7 @@ def _result(prog, meta, o, names, N):
     if prog.spawn is not None:
         stats.update((n, o.stats[ST[n]]) for n in ("spawned", "children_dropped", "children_truncated"))
     ys, trunc = _split_ys(prog, list(o.ys))
-    trunc, stats["n_truncated"] = _truncation(trunc, o.n_truncated, N)
+    trunc, stats["n_truncated"] = _truncation(trunc, o, N)
     _record_outputs(prog, o, res_out, stats)
     return Result(res_out, unflatten(meta["ytree"], ys), trunc, stats)
 
@@ -595,14 +595,16 @@ def _sum_outputs(prog, o, names):
     return {n: o.tallies[at[tn.index(n)]].reshape(prog.tallies[tn.index(n)].shape) for n in names if n in tn}
 
 
-def _truncation(trunc, ntr, N):
+def _truncation(trunc, o, N):
     """Result.truncated and stats['n_truncated']: without max_steps no item is truncated (bool[N] zeros, an int32
     zero), as in the reference (_api.py:689-693)."""
     if trunc is not None:
-        return trunc, ntr
+        return trunc, o.n_truncated
     import torch
-    z = torch.zeros((1 + (N + 3) // 4,), dtype=torch.int32, device="cuda")        # (one fill for both)
-    return z[1:].view(torch.bool)[:N], z[0]
+    z = torch.zeros((N,), dtype=torch.bool, device="cuda")
+    # (without a cap the launch counts no truncated children either: its zero, of a buffer of 20 bytes and not of z,
+    # which a kept count would keep)
+    return z, o.stats[ST["children_truncated"]]
 
 
 def _record_outputs(prog, o, res_out, stats):
@@ -1302,7 +1304,7 @@ def _run_tangents(mapped, args, tans, lanes, n_active=None, wide=False):
     stats = {n: o.stats[ST[n]] for n in ("fixed_point_overflow", "dropped_emits")}
     if prog.spawn is not None:
         stats.update((n, o.stats[ST[n]]) for n in ("spawned", "children_dropped", "children_truncated"))
-    trunc, stats["n_truncated"] = _truncation(trunc, o.n_truncated, N)
+    trunc, stats["n_truncated"] = _truncation(trunc, o, N)
     t_tal = [dict() for _ in range(lanes)]
     if rs:
         bad, over, offs = _tree_records(o, recs, prog, stats)

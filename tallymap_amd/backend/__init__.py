@@ -196,7 +196,7 @@ def launch_noalloc(c, ins, N, stream=None):
 
     import torch
     L = c.layout
-    if getattr(L, "aux", None) or getattr(L, "r_q", None) or not getattr(L, "scratch", None):
+    if getattr(L, "aux", None) or getattr(L, "r_q", None) or not L.n_claim:
         raise ValueError("tallymap_amd: launch_noalloc runs plain forward programs (no Records, no spawn)")
     scr = set(L.scratch)
     outs, slots, nbytes = [], [], []
@@ -321,7 +321,7 @@ def _run_spawn(c, prog, ins, N):
                 ops.append(z)
         else:
             ops = cur[:nP]
-        ctl[K.SHARD0:].zero_()                         # the item claim counters
+        ctl[K.SHARD0:L.n_claim].zero_()                # the item claim counters
         ctl[32:34].zero_()                             # the ticket counter
         gen = list(outs)
         for r, t in zip(L.r_q, spare):
@@ -423,7 +423,7 @@ def run_generations(prog, gens, bc, opts):
     for g, (ops, n) in enumerate(gens):
         ins = [device_tensor(x, a.dtype) for x, a in zip(ops, prog.p_avals())]
         if g:
-            outs[L.r_ctl - base].view(torch.int32)[K.SHARD0:].zero_()     # (the item claim counters, per launch)
+            outs[L.r_ctl - base].view(torch.int32)[K.SHARD0:L.n_claim].zero_()     # (the item claim counters, per launch)
         _queue(c, ins + b_ins, outs, n, L.n_zero if g == 0 else 0, 0)
     _queue(c, [device_tensor(x, a.dtype) for x, a in zip(gens[0][0], prog.p_avals())] + b_ins, outs, 0, 0, L.flags)
     tallies = [outs[L.r_out[k] - base] for k in prog.out_tallies]

@@ -6,7 +6,8 @@ every N):
     results [sum tallies][exact scratch of each exact tally][ctl u32][stats i32[5]] | [per-item results]
 The first group of results (up to stats) is zeroed by tm_zero before tm_main runs: the reference's n_zero
 (reference backends/kernel/kernel.py:565-591, shim.cc:215-218).  ctl holds the count of truncated items
-(word 2) and the claim counters of the item ranges.
+(word 2), the claim counters of the item ranges and, where steps are computed ahead, float64 sums of the privatised
+float32 tallies, which tm_post rounds into them.
 
 tm_main is the hand-written CDNA4 loop (reference kernel.py:812-838 is the CUDA one it replaces):
   * a persistent grid (256 CUs x achieved occupancy), block BLOCK = 256 (4 wave64s);
@@ -88,7 +89,7 @@ class Layout:
     r_ctl: int
     r_stats: int
     r_ys: list
-    flags: int             # bit1: launch tm_post
+    flags: int             # bit 1: launch tm_post; bit 3: launch it where the launch spread
     mode: str
     priv: list
     zero_words: list       # (buffer index, u32 words) zeroed by tm_zero
@@ -98,8 +99,11 @@ class Layout:
     aux: list = dataclasses.field(default_factory=list)
     # spawn: the next generation's per-item operand buffers (result indices, one per per-item operand, Q rows)
     r_q: list = dataclasses.field(default_factory=list)
-    # the buffers only the kernels read (exact / fixed-point words, ctl): what tm_launch_noalloc may place itself
+    # the buffers only the kernels read (exact / fixed-point words, ctl without float64 sums): what tm_launch_noalloc
+    # may place itself
     scratch: list = dataclasses.field(default_factory=list)
+    # u32 words of ctl up to the end of its claim counters (0: a program without them); float64 sums may follow
+    n_claim: int = 0
 
 
 def _split(jx):
@@ -468,7 +472,6 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     tape_w = int(getattr(prog, "tape_words", 0) or 0)
     tape_ck = int(getattr(prog, "tape_ck_words", 0) or 0)     # (the residual tape's checkpoint after the slots)
     r_tape = result((tape_w,), np.uint32, per_item=("itape",)) if tape_w else None
-    R = n_in + len(res)
 
     # ------------------------------------------------------------------------------- privatisation plan
     priv = []
@@ -1055,9 +1058,22 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 if not recs else None
             tail_lines = tail_ahead(pl_ahead) if pl_ahead is not None else step(5, False)
 
+    # A small launch of a program with steps computed ahead spreads to up to 512 workgroups, each of which adds its sum
+    # of a privatised float32 tally to the launch's: in float32 that many roundings lose what the float64 bins kept
+    # (quickstart at 10,000 items, error against float64: 1.0e-7 in 40 workgroups, 3.1e-7 in 512).  Such a program sums
+    # them in float64, and tm_post rounds once
+    # (in ctl, past the claim counters: no pointer of their own through the step loop)
+    wide, n_claim = {}, n_ctl
+    for k in priv:
+        s = prog.tallies[k]
+        if pl_ahead and s.dtype == C.F32 and not s.exact and not s.fixed:
+            wide[k] = n_ctl // 2
+            n_ctl += 2 * s.S
+    res[r_ctl - n_in] = ((n_ctl,), np.dtype(np.uint32), False)
+
     # ------------------------------------------------------------------------------------ assemble
     from . import compile as Cm
-    src = [Cm.prelude(), f"struct TmParams {{ void* p[{R}]; }};",
+    src = [Cm.prelude(), f"struct TmParams {{ void* p[{n_in + len(res)}]; }};",
            f"#define TM_STATS ((i32*)P.p[{r_stats}])", f"#define TM_CTL ((u32*)P.p[{r_ctl}])",
            f"#define TM_BLOCK {block}u"]
     if pl_ahead:
@@ -1098,6 +1114,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         elif s.fixed:
             post.append(_wide_readout(s, f"((const u64*)P.p[{r_scr[k]}])", f"((const i32*)P.p[{r_scr[k]}] + {2 * s.S})",
                                       f"((const u32*)P.p[{r_scr[k]}] + {3 * s.S})", f"P.p[{r_out[k]}]"))
+        elif k in wide:
+            post.append(f"for (i64 i = g; i < {s.S}; i += st) {{ float* const o = &((float*)P.p[{r_out[k]}])[i]; "
+                        f"*o = (float)((double)*o + ((const double*)P.p[{r_ctl}])[{wide[k]} + i]); }}")
     poison = [k for k in outs if prog.tallies[k].dtype in (C.F32, C.F64) and k not in raw]
     bad = ["TM_CTL[2] != 0u"] if prog.trunc is not None else []
     # a Records output past its capacity poisons every float output of the call (reference _api.py:120-131)
@@ -1125,7 +1144,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 post.append(f"if (TM_CTL[2] != 0u) for (i64 i = g; i < n_items * {n}; i += st) "
                             f"(({ctype(a.dtype)}*)P.p[{r_ys[j]}])[i] = __builtin_nanf(\"\");")
     if post:
-        flags |= 2
+        # (nothing but the float64 sums to read out: only where the launch spread, which tm_launch knows)
+        flags |= 8 if len(post) == len(wide) else 2
         src.append("extern \"C\" __global__ void tm_post(const TmParams P, const i64 n_items) {\n"
                    "  const i64 g = (i64)blockIdx.x * blockDim.x + threadIdx.x, st = (i64)gridDim.x * blockDim.x;\n  "
                    + "\n  ".join(post) + "\n}")
@@ -1512,6 +1532,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         src.append(f"#define TM_CN{k}(e) ({copy_of('(e)', ccopy[k])})")
     if priv:
         body.append("  __syncthreads();")
+        if wide:               # (a spread launch: more workgroups than its items fill)
+            body.append(f"  const bool tm_wide = (u64)tm_grid * TM_BLOCK >= (u64)n_items + TM_BLOCK;")
         for k in priv:
             s = prog.tallies[k]
             if s.exact:
@@ -1538,13 +1560,21 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {ct} x = tm_sh{k}[i]; "
                             f"if (x != 0) tm_gadd_u64(&((u64*)P.p[{r_out[k]}])[i], (u64)x); }}")
             elif s.dtype == C.F32:
-                body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const float x = (float){sum_copies(f'tm_sh{k}', ncopy.get(k, 1))}; "
-                            f"if (x != 0.0f) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], x); }}")
+                gw = f"(double*)tm_ctr + {wide[k]} + i" if k in wide else None
+                go = f"&((float*)P.p[{r_out[k]}])[i]"
+
+                def flush(total, cond, x32, x64):
+                    """add bin i's total of the workgroup to the launch's."""
+                    add = f"tm_gadd_f32({go}, {x32});"
+                    if gw is not None:
+                        add = f"{{ if (tm_wide) tm_gadd_f64({gw}, {x64}); else {add} }}"
+                    body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {total}; if ({cond}) {add} }}")
+                flush(f"{'double' if k in d64 else 'float'} x = {sum_copies(f'tm_sh{k}', ncopy.get(k, 1))}", "x != 0.0f",
+                      "(float)x", "x")
                 for (kk, _), (nm, c) in counts.items():
                     if kk == k:
-                        body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const u64 n = {sum_copies(nm, ccopy[k])}; "
-                                    f"if (n != 0ull) tm_gadd_f32(&((float*)P.p[{r_out[k]}])[i], "
-                                    f"tm_u64_f32(n) * {lit(c, np.float32)}); }}")
+                        flush(f"u64 n = {sum_copies(nm, ccopy[k])}", "n != 0ull", f"tm_u64_f32(n) * {lit(c, np.float32)}",
+                              f"(double)n * {lit(c, np.float64)}")
             else:
                 ct = ctype(s.dtype)
                 body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {ct} x = tm_sh{k}[i]; "
@@ -1574,5 +1604,5 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                flags=flags, mode=mode, priv=priv, zero_words=zero_words, r_q=r_q,
                records=[dict(name=ri["name"], capacity=ri["capacity"], r_ctr=(r_rctr, RC_WORDS // 2 * ri["ctr"] + RC_TOTAL),
                              fields={f: rr for f, (_, rr) in ri["fields"].items()}) for ri in rec_info], aux=aux,
-               scratch=sorted(r_scr.values()) + [r_ctl])
+               scratch=sorted(r_scr.values()) + ([] if wide else [r_ctl]), n_claim=n_claim)
     return "\n".join(src) + "\n", L

@@ -448,7 +448,7 @@ TM_DFN void tm_ladd_f32(float* a, float v) {          // a: LDS
   else if (!TmAddF32::zero(v)) TmAddF32::cas<__HIP_MEMORY_SCOPE_WORKGROUP>(a, v);
 }
 TM_DFN void tm_gadd_f64(double* a, double v) {
-  if (!TmAddF64::small(v)) unsafeAtomicAdd(a, v);
+  if (!TmAddF64::small(v)) __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   else if (!TmAddF64::zero(v)) TmAddF64::cas<__HIP_MEMORY_SCOPE_AGENT>(a, v);
 }
 TM_DFN void tm_ladd_f64(double* a, double v) {

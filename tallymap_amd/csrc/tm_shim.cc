@@ -303,7 +303,7 @@ int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, 
   if (!g_hip_ok) return fail("tallymap_rocm: tm_init was not called");
   if (n < 1 || block < 64 || block > 1024 || block % 64) return fail("tallymap_rocm: bad launch shape");
   if (n_items < 0) return fail("tallymap_rocm: negative item count");
-  if ((flags & 4) && (n_zero > 0 || (flags & 2)))
+  if ((flags & 4) && (n_zero > 0 || (flags & (2 | 8))))
     return fail("tallymap_rocm: flags bit 4 (a later spawn generation) runs tm_main alone");
   std::shared_ptr<Loaded> L;
   if (loaded(id, &L)) return 1;
@@ -324,8 +324,10 @@ int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, 
   memcpy(args.data() + sizeof(void*) * n, &karg, sizeof(long long));
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (n_zero > 0 && L->zero && launch1(L->zero, 64, 256, s, args, "tm_zero")) return 1;
+  bool spread = n_items == 0;       // (no tm_main: what earlier launches into these buffers left)
   if (n_items > 0) {
     long long want = (n_items + block - 1) / block;
+    const long long full = want;
     const long long cap = (long long)L->cus * occ;
     if (L->spread > 1 && want < cap) {
       // Fewer items than resident lanes: tm_spread lanes per item, up to 8 waves per CU (2 per SIMD), and a wave per
@@ -336,6 +338,7 @@ int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, 
       want = std::max({want, std::min(wide, (long long)L->cus * 512 / block), std::min(wave, (long long)L->cus)});
     }
     const unsigned grid = (unsigned)(want < cap ? want : cap);
+    spread = grid > full;
     if (launch1(L->main, grid, block, s, args, "tm_main")) return 1;
     std::lock_guard<std::mutex> lk(g_mu);
     if (!L->block0) {
@@ -343,7 +346,7 @@ int tm_launch(long long id, void* stream, void* const* bufs, int n, int n_zero, 
       L->occ0 = occ;
     }
   }
-  if ((flags & 2) && L->post && launch1(L->post, 64, 256, s, args, "tm_post")) return 1;
+  if (((flags & 2) || ((flags & 8) && spread)) && L->post && launch1(L->post, 64, 256, s, args, "tm_post")) return 1;
   return 0;
 }
 

@@ -149,3 +149,30 @@ def test_steps_with_loops_of_their_own(oracle, name):
     k, y = _host_steps(oracle, name, steps, x, keys)
     assert np.array_equal(r.per_item[0].cpu().numpy(), k)
     assert np.array_equal(r.per_item[1].cpu().numpy(), y)
+
+
+@pytest.mark.parametrize("n", [1, 40, 1000, 9001])
+def test_a_spread_launchs_float_sums_round_once(oracle, n):
+    """the sums of up to 512 workgroups into a float32 bin: the float64 sum of the emitted values (each one of them
+    representable, positive: float64's own roundings are far below) rounded once to float32, also for a constant, in
+    a register-held, a float64 and a float32 LDS tally."""
+    sizes = {"one": 1, "few": 5, "many": 1500}
+
+    def item(t, key):
+        def body(c):
+            k, t = c
+            u = random.uniform(random.fold_in(key, k), minval=0.25, maxval=1.75)
+            for name, S in sizes.items():
+                t = t.add(name, k % S, u)
+            return k + 1, t.add("c", 0, 0.1)
+        return lax.while_loop(lambda c: c[0] < 4, body, (np.int32(0), t))[1]
+    keys = np.asarray(random.split(random.PRNGKey(5), n))
+    r = tm.vmap(item, outputs={**{k: tm.Sum((S,)) for k, S in sizes.items()}, "c": tm.Sum((1,))}, in_axes=(0,))(keys)
+    u = np.array([[oracle.uniform(oracle.fold_in(key, k), 0.25, 1.75) for k in range(4)] for key in keys], np.float64)
+    want = {k: np.bincount(np.arange(4) % S, weights=u.sum(0), minlength=S) for k, S in sizes.items()}
+    want["c"] = np.array([4 * n * float(np.float32(0.1))])
+    for k, w in want.items():
+        got = r.outputs[k].cpu().numpy().astype(np.float64)
+        # (the float32 LDS bins: a rounding per add within a workgroup, at most 16 items' there)
+        slack = 2.0 ** -24 * (16 if k == "many" else 1) + 1e-12
+        assert np.all(np.abs(got - w) <= slack * w), (n, k, got[:5], w[:5])

@@ -148,3 +148,13 @@ def test_c1_many_chunks_per_wave(oracle):
     assert np.array_equal(_np(res.per_item), ref.per_item)
     ok, err = _close(_np(res.outputs["hist"]), ref.tallies64["hist"])
     assert ok, err
+
+
+@pytest.mark.parametrize("n", [1, 3, 1001, 100_000])
+def test_a_kept_count_does_not_keep_the_calls_buffers(n):
+    """stats['n_truncated'] of a call without max_steps: a zero that holds no per-item memory."""
+    import torch
+    r = tm.vmap(lambda t, x: t.add("h", 0, x), outputs={"h": tm.Sum((1,))}, in_axes=(0,))(np.ones(n, np.float32))
+    assert r.truncated.shape == (n,) and r.truncated.dtype == torch.bool and not bool(r.truncated.any())
+    c = r.stats["n_truncated"]
+    assert c.dtype == torch.int32 and c.shape == () and int(c) == 0 and c.untyped_storage().nbytes() <= 64
