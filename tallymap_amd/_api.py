@@ -653,7 +653,8 @@ def vmap(fn=None, *, outputs, in_axes=0, max_steps=None, spawn=None, backend="au
                (how vjp, grad and value_and_grad differentiate w.r.t. broadcast arguments: 'auto', the default,
                runs one forward launch with a tangent lane per differentiated element when every differentiated
                argument is broadcast, they hold at most 8 float32 elements and a loop carry needs the reverse
-               sweep, else the replay adjoint; 'reverse' always the replay adjoint; 'tangent' lanes whenever the
+               sweep (or, with exact sums, in a vjp of 2^19 items or more where that launch costs less than the
+               forward and the adjoint), else the replay adjoint; 'reverse' always the replay adjoint; 'tangent' lanes whenever the
                arguments are broadcast); blocks_per_cu (at most this many workgroups per CU in the item loop's
                persistent grid; default: the occupancy, and 2 for a spawning call, whose shower ran 13 % faster
                at 2 than at 8); min_blocks_per_sm (workgroups per CU the compiler must leave registers for:
@@ -849,9 +850,10 @@ def vjp(mapped, *args, argnums=None, n_active=None):
     Where the gradient runs as tangent lanes (option grad_mode; by default a few broadcast elements through a loop
     carry, or, in large calls, where one launch of them costs less than the forward and the adjoint), the forward call
     is the jvp launch with one lane per differentiated element and the pullback is a contraction of its tangent
-    outputs with the cotangents, on the device, with no launch of its own (plain float32 tallies' tangents accumulate
-    in float64 atomics: reproducible to float64 reassociation; grad_mode='reverse' gives the replay adjoint's exact,
-    bitwise reproducible broadcast cotangents)."""
+    outputs with the cotangents, on the device, with no launch of its own (through a loop carry, plain float32 tallies'
+    tangents accumulate in float64 atomics: reproducible to float64 reassociation; grad_mode='reverse' gives the replay
+    adjoint's exact, bitwise reproducible broadcast cotangents.  Where the lanes replace a forward-only adjoint, their
+    sums are exact and as reproducible as its)."""
     m = mapped._sized(args, n_active)
     prog, meta, pi, bc, N, axes = m._prepare(args)
     tg = _tangent_plan(m, prog, args, axes, argnums,
@@ -1064,8 +1066,8 @@ _TPLAN = collections.OrderedDict()   # (program, argnums, axes, mode, argument t
 
 def _tangent_plan(m, prog, args, axes, argnums, pair=False):
     """how the gradient w.r.t. argnums is computed (option grad_mode): None for the replay adjoint (reverse mode),
-    else (spec, wrt, lanes, bav) with lanes = [(broadcast operand, flat element)], one forward-mode tangent lane per
-    float32 element of the broadcast arguments (bav: the program's broadcast operand avals).
+    else (spec, wrt, lanes, bav, wide) with lanes = [(broadcast operand, flat element)], one forward-mode tangent lane
+    per float32 element of the broadcast arguments (bav: the program's broadcast operand avals; wide: jvp_program's).
 
     The gradient of a tally's <ct, T> w.r.t. a broadcast parameter theta of P elements is sum_k ct[k] dT[k]/dtheta:
     P directional derivatives, which one forward launch computes as P tangent lanes beside the primal (jvp), for
@@ -1076,7 +1078,8 @@ def _tangent_plan(m, prog, args, axes, argnums, pair=False):
     adjoint is a recording forward, a canonical ordering and a count and a reverse launch per generation; the lanes
     are one forward through the generations, the children carrying their parents' tangents).  pair: the caller needs
     the forward's outputs before the cotangent (vjp), so a forward-only adjoint is a second launch after the
-    forward's; the lanes are taken where one launch of them costs less (_lanes_beat_pair).  'reverse' always
+    forward's; the lanes are taken where one launch of them costs less (_lanes_beat_pair), with exact sums as the
+    adjoint's, so that a gradient is reproducible at every size.  'reverse' always
     replays; 'tangent' takes the lanes whenever the arguments allow (any P, 16 lanes per launch).  Per-item
     arguments and Records outputs always replay."""
     mode = m._opts.get("grad_mode") or "auto"
@@ -1095,35 +1098,52 @@ def _tangent_plan(m, prog, args, axes, argnums, pair=False):
     return plan
 
 
-LANES_PAIR = 0.75              # vjp takes lanes for a forward-only adjoint when a lane step costs at most this share of a
-                               # forward step and an adjoint step together (kernel.cost): the random walk problem's
-                               # three lanes are 0.60 of them, and its loss gradient at 4,194,304 items took 1,156 us by
-                               # the two launches against 610 by one ...
+LANES_PAIR = 0.85              # vjp takes lanes for a forward-only adjoint when a lane step costs at most this share of a
+                               # forward step and an adjoint step together (kernel.cost, an exact emit at 30): the
+                               # random walk problem's three lanes are 0.80 of them, and its loss gradient at 4,194,304
+                               # items took 1,179 us by the two launches against 919 by one; the quickstart's lane is
+                               # 0.58 (661 against 400), walk on spheres' five 0.55 (at 1,048,576: 514 against 358) ...
+LANES_PAIR_BINS = 16           # ... and every tangent is emitted into at least this many bins: the lanes of a wave that
+                               # add to one exact bin take turns (up-and-out calls, eight lanes onto one and eight bins,
+                               # at 1,048,576: 3,903 by the two launches against 4,465) ...
 LANES_PAIR_ITEMS = 1 << 19     # ... in calls of at least this many items: the contraction with the cotangent is ~60 us of
-                               # small device operations (the same gradient at 1,100,000 items: 422 us against 238, at
-                               # 100,000 126 against 184)
+                               # small device operations against a launch that grows with the items' steps, which are
+                               # not known (at 524,288 items: the walk of ~130 steps 4,234 us by two launches against
+                               # 2,301, walk on spheres 391 against 262, random walk 320 against 286, but the quickstart
+                               # of ~8 steps 130 against 181; at 1,048,576 that is 228 against 188)
 
 
 def _lanes_beat_pair(prog, wrt, nlanes):
     """whether one launch of the program with its tangent lanes costs less than the forward launch and the forward-only
-    adjoint's: by the static cost of a step of each (kernel.cost), and only where every float32 output's tangent is
-    held in float64 in LDS (a larger tally's float32 global atomics would cost precision and time)."""
+    adjoint's: by the static cost of a step of each (kernel.cost), and only where every tangent is an exact sum in LDS
+    (the adjoint's sums are exact) and none is a per-item result's."""
     from . import backend as B
     from .backend import kernel as K
     from .backend import reverse as R
     from .backend import simplify
     if K._split(prog.jaxpr) is None:
         return False
-    q = _jvp_prog(prog, (False,) * prog.nP, tuple(i in wrt[1] for i in range(prog.nB)), nlanes, True)
-    if any(t.kind == "sum" and t.dtype == C.F32 and not t.exact for t in q.tallies[prog.nT:]):
+    q = _jvp_prog(prog, (False,) * prog.nP, tuple(i in wrt[1] for i in range(prog.nB)), nlanes, "exact")
+    if q.tangent_ys:           # (their tangents are N x lanes values that the adjoint does not store)
         return False
+    L = K.build(q)[1]
+    for k in L.emitted:
+        if k >= prog.nT and not (q.tallies[k].exact and k in L.priv and q.tallies[k].S >= LANES_PAIR_BINS):
+            return False
     adj, pl = B._adjoint(prog, wrt)
 
     def step(p):
+        """(cost of a step, its emits)"""
         at = K._split(p.jaxpr)
-        return None if at is None else K.cost(simplify.cse(p.jaxpr.eqns[at].params["body_jaxpr"]).eqns)
+        if at is None:
+            return None
+        eqns = simplify.cse(p.jaxpr.eqns[at].params["body_jaxpr"]).eqns
+        return K.cost(eqns), sum(e.prim == "tallymap_emit" for e in C.walk_eqns(C.Jaxpr([], [], eqns)))
     costs = [step(p) for p in (q, prog, R.forward_only_program(adj, pl))]
-    return None not in costs and costs[0] <= LANES_PAIR * (costs[1] + costs[2])
+    if None in costs:
+        return False
+    (lane, ne), (fwd, n0), (back, _) = costs
+    return lane + 24 * (ne - n0) <= LANES_PAIR * (fwd + back)
 
 
 def _tangent_plan_of(prog, args, axes, an, mode, pair):
@@ -1138,13 +1158,13 @@ def _tangent_plan_of(prog, args, axes, an, mode, pair):
     if mode == "tangent":
         if why is not None:
             raise UnsupportedError(f"tallymap: grad_mode='tangent': {why}")
-        return (spec, wrt, lanes, bav) if lanes else None
+        return (spec, wrt, lanes, bav, True) if lanes else None
     if why is not None or not lanes or len(lanes) > TANGENT_MAX:
         return None
     from . import backend as B
-    if prog.spawn is None and not B.needs_sweep(prog, wrt) and not (pair and _lanes_beat_pair(prog, wrt, len(lanes))):
-        return None
-    return spec, wrt, lanes, bav
+    if prog.spawn is not None or B.needs_sweep(prog, wrt):
+        return spec, wrt, lanes, bav, True
+    return (spec, wrt, lanes, bav, "exact") if pair and _lanes_beat_pair(prog, wrt, len(lanes)) else None
 
 
 def _unit(shape, dt, e):
@@ -1180,7 +1200,7 @@ def _tangent_vjp(m, args, plan, n_active):
     differ in the rounding of the items' float32 derivatives only.  A truncated item, or in a spawning call a
     dropped or truncated child, makes every cotangent NaN, as the replay and tree adjoints do."""
     import torch
-    spec, wrt, lanes, bav = plan
+    spec, wrt, lanes, bav, wide = plan
     primal, t_tal, t_ys = None, [], []
     for s in range(0, len(lanes), MAX_LANES):
         chunk = lanes[s:s + MAX_LANES]
@@ -1194,7 +1214,7 @@ def _tangent_vjp(m, args, plan, n_active):
                 leaves = [_unit(sh, bav[k].dtype, e) if k == i else None for k, sh in zip(idx, shapes)]
                 per.append(unflatten(td, leaves) if td is not None else leaves[0])
             tans[pos] = per
-        pr, tt, ty, _ = _run_tangents(m, args, tans, len(chunk), n_active, wide=True)
+        pr, tt, ty, _ = _run_tangents(m, args, tans, len(chunk), n_active, wide=wide)
         primal = pr if primal is None else primal
         t_tal += tt
         t_ys += ty
@@ -1263,7 +1283,8 @@ def _match_leaves(prim, tan):
 def _run_tangents(mapped, args, tans, lanes, n_active=None, wide=False):
     """one launch of the jvp program with `lanes` directions.  tans[pos]: None or a list of `lanes` tangent arrays
     for positional argument pos (its shape) -> (primal Result, per lane {name: tangent tally}, per lane [tangents
-    of the float per-item results (None for the others)]).  wide: plain float32 tallies' tangents in float64."""
+    of the float per-item results (None for the others)]).  wide: plain float32 tallies' tangents in float64 (True) or
+    exact, rounded to float64 ('exact')."""
     from . import backend as B
     mapped = mapped._sized(args, n_active)
     prog, meta, pi, bc, N, axes = mapped._prepare(args)

@@ -104,6 +104,7 @@ class Layout:
     scratch: list = dataclasses.field(default_factory=list)
     # u32 words of ctl up to the end of its claim counters (0: a program without them); float64 sums may follow
     n_claim: int = 0
+    emitted: set = dataclasses.field(default_factory=set)      # the tally slots with an emit
 
 
 def _split(jx):
@@ -506,7 +507,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     ncopy, room = {}, 0 if lean else LDS_F64 // 8
     for k in priv:
         s = prog.tallies[k]
-        if k in d64 or (s.dtype == C.F64 and not s.fixed):
+        if k in d64 or (s.dtype == C.F64 and not s.fixed and not s.exact):
             ncopy[k] = copies(s.S, room)
             room -= s.S * ncopy[k] if ncopy[k] > 1 else 0
 
@@ -523,6 +524,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     counts = {}                 # (tally slot, f32 bits of a constant emitted value) -> (LDS u64 counter array, value)
     rcounts = {}                # the same, for a lane-register tally: -> (the lane's u32 counter names per bin, value)
 
+    emitted = set()             # the slots an emit was written for (a tangent that is always zero has none)
     quiet = set(getattr(prog, "quiet_tallies", ()))
     lead = [False]              # emitting the update side of a group of lanes (tail loop)
 
@@ -532,6 +534,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         s = prog.tallies[k]
         if s.kind == "discard":
             return t
+        emitted.add(k)
         ei = em_.bind(idx.el[0], np.int32, "ei")
         ok = em_.bind(f"(u32){ei} < {s.S}u", C.BOOL, "ok")
         if lead[0]:            # (a group of lanes holds the item: one of them emits)
@@ -1106,6 +1109,11 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         if s.exact:
             words = f"((const u64*)P.p[{r_scr[k]}])"
             fl = f"((const u32*)P.p[{r_scr[k]}] + {2 * XW * s.S})"
+            if s.dtype == C.F64:   # (a tangent's exact sum: not among the call's outputs, so none of its overflows)
+                post.append(f"for (i64 i = g; i < {s.S}; i += st) ((double*)P.p[{r_out[k]}])[i] = "
+                            f"(({fl}[i >> 5] >> (i & 31)) & 1u) != 0u ? __builtin_nan(\"\") : "
+                            f"tm_xread_f64(&{words}[i * {XW}]);")
+                continue
             post.append(f"for (i64 i = g; i < {s.S}; i += st) {{ bool bad = false; "
                         f"const float o = tm_xread(&{words}[i * {XW}], &bad); "
                         f"const bool f = (({fl}[i >> 5] >> (i & 31)) & 1u) != 0u; "
@@ -1604,5 +1612,6 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                flags=flags, mode=mode, priv=priv, zero_words=zero_words, r_q=r_q,
                records=[dict(name=ri["name"], capacity=ri["capacity"], r_ctr=(r_rctr, RC_WORDS // 2 * ri["ctr"] + RC_TOTAL),
                              fields={f: rr for f, (_, rr) in ri["fields"].items()}) for ri in rec_info], aux=aux,
-               scratch=sorted(r_scr.values()) + ([] if wide else [r_ctl]), n_claim=n_claim)
+               scratch=sorted(r_scr.values()) + ([] if wide else [r_ctl]), n_claim=n_claim,
+               emitted=emitted)
     return "\n".join(src) + "\n", L

@@ -566,6 +566,15 @@ TM_FN float tm_xread(const u64* a, bool* bad) {
   return neg ? -f : f;
 }
 
+// the same words rounded once to f64 (their range, below 2^320 units of 2^-149, is within f64's)
+TM_FN double tm_xread_f64(const u64* a) {
+  u32 d[TM_XW + 2];
+  const bool neg = tm_canon_digits((const i64*)a, TM_XW, d);
+  if (neg) tm_negate_digits(d, TM_XW + 2);
+  const double f = tm_digits_f64(d, TM_XW + 2, -149);
+  return neg ? -f : f;
+}
+
 // --------------------------------------------------------------------- the scaled fixed-point sum (WIDE)
 // A bin is an int64 low word (wrapping) and an i32 word counting its signed wraps: an add of q that takes the low
 // word out of the int64 range (tm_wraps on the old value the atomic returns) adds sign(q) to the count, so the

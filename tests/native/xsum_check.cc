@@ -2,8 +2,8 @@
 // infrastructure).  Modes (argv[1]):
 //   (none)  reads f32 values (one hex word per line on stdin), emits them into one bin with tm_xemit_with (a plain
 //           add standing in for the device's int64 atomic), prints the readout's bits and the flag;
-//   words   reads TM_XW int64 words (hex, two's complement) of one bin, prints tm_xread's bits and its flag: the
-//           readout of words that are not canonical (any signed values, as concurrent carries leave them);
+//   words   reads TM_XW int64 words (hex, two's complement) of one bin, prints tm_xread's bits, its flag and
+//           tm_xread_f64's bits: the readout of words that are not canonical (any signed values, as concurrent carries leave them);
 //   wide    reads pairs (low word hex u64, count decimal i32), prints tm_wide_f64's bits for each.
 #include <cstdio>
 #include <cstdint>
@@ -22,7 +22,7 @@ int main(int argc, char** argv) {
       if (scanf("%llx", &w[j]) != 1) return 2;
     bool bad = false;
     const float r = tm_xread(w, &bad);
-    printf("%08x %d\n", tm_f2u(r), (int)bad);
+    printf("%08x %d %016llx\n", tm_f2u(r), (int)bad, (unsigned long long)tm_d2u(tm_xread_f64(w)));
     return 0;
   }
   if (!strcmp(mode, "wide")) {

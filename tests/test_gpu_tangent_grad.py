@@ -171,3 +171,45 @@ def test_value_and_grad_by_lanes_and_truncation():
     gt = tm.grad(ft, argnums=1)(keys, mu_a)
     _sync()
     assert np.isnan(float(_np(gt)))
+
+
+def test_large_vjp_by_one_launch_is_reproducible():
+    """vjp of a program whose adjoint is a second launch, in a call large enough that the lanes replace both: the same
+    bits every run, as the exact adjoint's on either side of that size, and its value."""
+    p = PB.PROBLEMS["random_walk"]
+    for n in (tm._api.LANES_PAIR_ITEMS - 1, tm._api.LANES_PAIR_ITEMS + 3):
+        print(f"case: random walk vjp N={n}", flush=True)
+        args, extra = p["inputs"](n)
+        ct = p["ct"](PB.mapped("random_walk")(*args).outputs, n, extra)
+        got = [_np(tm.vjp(PB.mapped("random_walk"), *args, argnums=p["argnum"])[1](ct)) for _ in range(4)]
+        want = _np(tm.vjp(PB.mapped("random_walk", grad_mode="reverse"), *args, argnums=p["argnum"])[1](ct))
+        for g in got[1:]:
+            assert np.array_equal(g, got[0]), got
+        assert _close(got[0], want, MTOL)[0], (got[0], want)
+
+
+def test_exact_tangents_of_non_finite_values():
+    """a bin with a non-finite tangent makes the gradient that its cotangent reaches NaN, as the exact adjoint does, and
+    counts no overflow of an output's own."""
+    n = tm._api.LANES_PAIR_ITEMS
+
+    def item(t, x, th):
+        def body(c):
+            k, t = c
+            w = jnp.exp(jnp.sin(jnp.log(x) + k.astype(jnp.float32)))
+            return k + 1, t.add("h", k, th[0] * w)
+        return lax.while_loop(lambda c: c[0] < 2, body, (np.int32(0), t))[1]
+    x = np.linspace(0.25, 4.0, n).astype(np.float32)
+    th = np.array([1.5], np.float32)
+    f, fr = (tm.vmap(item, outputs={"h": tm.Sum((16,))}, in_axes=(0, None), **o) for o in ({}, {"grad_mode": "reverse"}))
+    m = f._sized((x, th), None)
+    prog, _, _, _, _, axes = m._prepare((x, th))
+    assert tm._api._tangent_plan(m, prog, (x, th), axes, 1, pair=True)[4] == "exact"
+    ct = {"h": np.linspace(1.0, -0.5, 16).astype(np.float32)}
+    for bad in (False, True):
+        x[7] = -1.0 if bad else x[7]               # (its logarithm is NaN)
+        res, pull = tm.vjp(f, x, th, argnums=1)
+        got, want = _np(pull(ct)), _np(tm.vjp(fr, x, th, argnums=1)[1](ct))
+        assert np.isnan(got[0]) == np.isnan(want[0]) == bad
+        assert bad or _close(got, want, MTOL)[0], (got, want)
+        assert int(res.stats["fixed_point_overflow"]) == 0

@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 import subprocess
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -96,7 +97,7 @@ def test_exact_accumulator_matches_python_integers(xsum):
 def _xwords(exe, w):
     inp = " ".join("%016x" % (int(x) & (2 ** 64 - 1)) for x in w)
     out = subprocess.run([exe, "words"], input=inp, capture_output=True, text=True, check=True).stdout.split()
-    return np.uint32(int(out[0], 16)).view(np.float32), out[1] == "1"
+    return np.uint32(int(out[0], 16)).view(np.float32), out[1] == "1", np.uint64(int(out[2], 16)).view(np.float64)
 
 
 def test_exact_accumulator_carries_between_words(xsum):
@@ -118,7 +119,7 @@ def test_exact_accumulator_carries_between_words(xsum):
 def test_exact_readout_of_arbitrary_words(xsum):
     """tm_xread on words that are not canonical (any int64 per word, as concurrent adds and carries leave them):
     the correctly rounded f32 of sum_j w_j 2^(32 j) units of 2^-149 -- Python integers -- with the flag exactly when
-    that total is beyond f32.  Covers signs that differ across words, totals near zero, ties and the top word."""
+    that total is beyond f32, and tm_xread_f64 its correctly rounded f64.  Covers signs that differ across words, totals near zero, ties and the top word."""
     rng = np.random.default_rng(5)
     lim = 2 ** 63
     cases = [[0] * 9, [1] + [0] * 8, [-1] + [0] * 8, [0] * 8 + [-1], [lim - 1] * 9, [-lim] * 9,
@@ -134,7 +135,8 @@ def test_exact_readout_of_arbitrary_words(xsum):
     for w in cases:
         total = sum(int(x) << (32 * j) for j, x in enumerate(w))
         want = X.round_units(total)
-        g, bad = _xwords(xsum, w)
+        g, bad, d = _xwords(xsum, w)
+        assert d == float(Fraction(total, 2 ** 149)) and (d != 0) == (total != 0), (w, d)
         assert bad == (want is None), (w, g)
         if want is not None:
             assert g.view(np.uint32) == want.view(np.uint32), (w, g, want)

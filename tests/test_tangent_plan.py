@@ -98,8 +98,9 @@ def test_auto_takes_lanes_for_a_spawning_call():
 
 def test_vjp_takes_lanes_where_they_cost_less_than_two_launches():
     """vjp needs the outputs before the cotangent: forward and forward-only adjoint are two launches, the lanes one.
-    Taken for small float32 sums and few elements; not where a tangent would leave float64 LDS sums (the disk's maps),
-    not with 'reverse', and grad / value_and_grad (one launch by the adjoint) stay."""
+    Taken for small float32 sums and few elements, with exact sums as the adjoint's; not where a tangent would leave LDS
+    (the disk's maps), goes to a few bins that a wave's lanes would wait for (up-and-out calls) or is a per-item
+    result's, not with 'reverse', and grad / value_and_grad (one launch by the adjoint) stay."""
     from tallymap_amd import problems
 
     def plan(f, args, argnum, pair):
@@ -109,8 +110,15 @@ def test_vjp_takes_lanes_where_they_cost_less_than_two_launches():
     rw = problems.PROBLEMS["random_walk"]
     args = rw["inputs"](64)[0]
     p = plan(problems.mapped("random_walk"), args, 2, True)
-    assert p is not None and p[2] == [(0, 0), (0, 1), (0, 2)]
+    assert p is not None and p[2] == [(0, 0), (0, 1), (0, 2)] and p[4] == "exact"
     assert plan(problems.mapped("random_walk"), args, 2, False) is None
+    assert plan(problems.mapped("barrier"), problems.PROBLEMS["barrier"]["inputs"](64)[0], 2, True) is None
+
+    def with_result(t, *a):
+        t, k = rw["item"](t, *a)
+        return t, (k, a[2][0] * 2.0)
+    f = tm.vmap(with_result, outputs=rw["outputs"], in_axes=rw["in_axes"])
+    assert plan(f, args, 2, True) is None
     assert plan(problems.mapped("random_walk", grad_mode="reverse"), args, 2, True) is None
     for cfg, inputs, pos in ((configs.c4_config(64), configs.c4_inputs(64), 3), (configs.C1, configs.c1_inputs(64), 0)):
         f = tm.vmap(cfg["item"], outputs=cfg["outputs"], in_axes=cfg["in_axes"], max_steps=cfg["max_steps"])
