@@ -348,6 +348,9 @@ TM_DFN i64 tm_qclaim(u64* ctr, bool when) {
   return when ? (i64)(b + tm_rank(m)) : -1;
 }
 
+// chunks of range s when nc chunks are dealt out to S ranges in turn
+TM_FN u64 tm_range(u64 nc, u32 s, u32 S) { return nc > s ? (nc - s + S - 1u) / S : 0ull; }
+
 // A Records output's slot claim (reference _tally.py:141-160): a wave takes raw slots from a private batch of TM_RB
 // consecutive slots, refilled with one atomic per TM_RB slots.  The batch state (base, slots left, records appended)
 // lives in the wave's LDS words, read by every active lane and written by the first, so lanes that diverged keep one

@@ -51,3 +51,27 @@ def test_active_items_only():
     for n, m in ((1000, 0), (1000, 1), (R + 5000, R), (R + 5000, R + 1), (2 * R, 7)):
         print("case: n", n, "active", m, flush=True)
         _check(n, n_active=m)
+
+
+def _doubling(t, x, i):
+    """x doubled i % 5 times, then added: the adjoint sweeps back over the steps, from a tape."""
+    x = lax.while_loop(lambda c: c[0] < i % 5, lambda c: (c[0] + 1, c[1] * 2.0), (np.int32(0), x))[1]
+    return t.add("h", i % 4, x)
+
+
+@pytest.mark.parametrize("opts", [dict(block=64, blocks_per_cu=1), dict(), dict(refill=8)], ids=str)
+def test_a_taped_gradient_runs_every_item_once(opts):
+    """the tape programs' ranges deal the chunks out in turn: one chunk per wave, the ranges' first and last ones, and
+    the last chunk of the call whole and short."""
+    import torch
+    f = tm.vmap(_doubling, outputs={"h": tm.Sum((4,))}, in_axes=(0, 0), **opts)
+    R = _resident(**opts)
+    for n in (1, 65, R, R + 1, R + 64, 2 * R + 4095, 2 * R + 4096, 2 * R + 4097, 3 * R - 63, 5 * R):
+        print("case:", opts, n, flush=True)
+        i = torch.arange(n, dtype=torch.int32, device="cuda")
+        x = 1.0 + (i % 7).float()
+        res, g = tm.value_and_grad(f, argnums=0)(x, i)
+        want = torch.pow(2.0, (i % 5).float())
+        assert torch.equal(g, want), n
+        h = torch.zeros(4, dtype=torch.float64, device="cuda").index_add_(0, i.long() % 4, (x * want).double())
+        assert torch.allclose(res.outputs["h"].double(), h, rtol=1e-5, atol=0.0), n
