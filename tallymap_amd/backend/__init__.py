@@ -150,7 +150,7 @@ def _alloc_specs(c, N):
         if per_item == ("itape",):
             outs.append(None)
             continue
-        if per_item == "tape":          # per launched lane (the launcher's persistent grid at this N)
+        if per_item == "tape":          # (rev_schedule='step') per launched lane: the persistent grid at this N
             sh = (_lanes(c, N),) + tuple(shape)
         elif isinstance(per_item, tuple) and per_item[0] == "rraw":
             # a Records raw buffer: the capacity and room for a partly used batch per launched wave
@@ -436,7 +436,10 @@ _LANES = {}
 
 
 def _lanes(c, N):
-    """the lanes tm_launch starts for c at N items: min(ceil(N / block), CUs x blocks per CU) x block."""
+    """the lanes tm_launch starts for c at N items: min(ceil(N / block), CUs x blocks per CU) x block.  A program with
+    steps computed ahead may start more (tm_spread): nothing of it is sized by its lanes."""
+    if c.layout.spread:
+        raise Cm.BackendError("internal: buffers sized by the lanes of a launch that spreads")
     r = _LANES.get(c.id)
     if r is None:
         r = _LANES[c.id] = kernel_info(c)["resident_threads"]

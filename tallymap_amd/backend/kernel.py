@@ -104,6 +104,7 @@ class Layout:
     scratch: list = dataclasses.field(default_factory=list)
     # u32 words of ctl up to the end of its claim counters (0: a program without them); float64 sums may follow
     n_claim: int = 0
+    spread: int = 0        # the module's tm_spread (0: its launches do not spread)
     emitted: set = dataclasses.field(default_factory=set)      # the tally slots with an emit
 
 
@@ -1057,6 +1058,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             em.close()
             return head, em.lines, len(words)
         if compact:
+            # (not with Records: their raw buffers are sized by the launch's lanes without the spread, _lanes)
             pl_ahead = Ahead.plan(we, lambda v: isinstance(v, C.Var) and isinstance(env.get(v.id), VTally), cost) \
                 if not recs else None
             tail_lines = tail_ahead(pl_ahead) if pl_ahead is not None else step(5, False)
@@ -1632,5 +1634,5 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                records=[dict(name=ri["name"], capacity=ri["capacity"], r_ctr=(r_rctr, RC_WORDS // 2 * ri["ctr"] + RC_TOTAL),
                              fields={f: rr for f, (_, rr) in ri["fields"].items()}) for ri in rec_info], aux=aux,
                scratch=sorted(r_scr.values()) + ([] if wide else [r_ctl]), n_claim=n_claim,
-               emitted=emitted)
+               emitted=emitted, spread=SPREAD if pl_ahead else 0)
     return "\n".join(src) + "\n", L

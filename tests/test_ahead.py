@@ -168,3 +168,32 @@ def test_a_condition_with_a_loop_runs_on_live_lanes_alone():
     assert cond.index("if (tm_live) {") < cond.index("while (true)")
     _, _, cond = _ahead_sides(loop_item("literal"))
     assert "if (tm_live)" not in cond
+
+
+def test_a_program_that_spreads_has_nothing_sized_by_its_lanes():
+    """Records' raw buffers have room for a batch per launched wave: no steps ahead there, and a size taken from a
+    spreading program's lanes is refused."""
+    import types
+
+    from tallymap_amd import backend as B
+    from tallymap_amd._api import Records
+
+    def item(rec):
+        def f(t, x, key):
+            def body(c):
+                k, x, t = c
+                u = random.uniform(random.fold_in(key, k))
+                t = t.append("r", {"u": u}) if rec else t.add("h", 0, u)
+                return k + 1, x * u, t
+            return lax.while_loop(lambda c: c[1] > 0.05, body, (np.int32(0), x, t))[2]
+        return f
+    for rec, out in ((False, {"h": Sum((1,))}), (True, {"r": Records({"u": np.float32}, 64)})):
+        src, L = K.build(_prog(item(rec), out, (0, 0), _walk_args(2)))
+        assert ("tm_spread" in src) == (L.spread > 0) == (not rec)
+        c = types.SimpleNamespace(layout=L, block=256, id=-7 - rec)
+        if L.spread:
+            with pytest.raises(B.Cm.BackendError, match="spreads"):
+                B._lanes(c, 100)
+        else:
+            B._LANES[c.id] = 1 << 20
+            assert B._lanes(c, 257) == 512 and B._lanes(c, 1 << 24) == 1 << 20
