@@ -1128,7 +1128,8 @@ def _lanes_beat_pair(prog, wrt, nlanes):
         return False
     L = K.build(q)[1]
     for k in L.emitted:
-        if k >= prog.nT and not (q.tallies[k].exact and k in L.priv and q.tallies[k].S >= LANES_PAIR_BINS):
+        t = q.tallies[k]       # (an exact sum rounded to float32 per bin would lose what bins of opposite signs cancel)
+        if k >= prog.nT and not (t.exact and t.dtype == C.F64 and k in L.priv and t.S >= LANES_PAIR_BINS):
             return False
     adj, pl = B._adjoint(prog, wrt)
 

@@ -298,8 +298,8 @@ def jvp_program(prog, pert_pi, pert_bc, lanes=1, wide=False):
     (a float32 LDS bin loses ~1e-4 relative over millions of them) carry no float32 accumulation error into the
     gradient by tangent lanes, which contracts in float64.  A tangent tally that would leave LDS in float64 keeps
     the primal's format: global float64 atomics cost more than the accuracy buys there (a large tally spreads its
-    emits over many bins).  wide='exact': such a tangent is the exact sum of its float32 emits, rounded once to float64,
-    where the exact words fit (the same bits every run, as the replay adjoint's cotangents have)."""
+    emits over many bins).  wide='exact': such a tangent, and an exact Sum's, is the exact sum of its float32 emits,
+    rounded once to float64, where the exact words fit (the same bits every run, as the replay adjoint's cotangents have)."""
     import dataclasses
 
     from ._api import ItemProgram, check_tallies
@@ -345,7 +345,7 @@ def jvp_program(prog, pert_pi, pert_bc, lanes=1, wide=False):
             t = dataclasses.replace(s, name=s.name + ("'" if lanes == 1 else f"'{l}"))
             if budget is not None and s.kind == "sum":
                 w = dataclasses.replace(t, dtype=C.F64, exact=wide == "exact")
-                if s.dtype == C.F32 and not s.exact and not s.fixed and tally_lds_bytes(w) <= budget:
+                if s.dtype == C.F32 and not s.fixed and (wide == "exact" or not s.exact) and tally_lds_bytes(w) <= budget:
                     t = w
                 if tally_lds_bytes(t) <= budget:
                     budget -= tally_lds_bytes(t)

@@ -213,3 +213,25 @@ def test_exact_tangents_of_non_finite_values():
         assert np.isnan(got[0]) == np.isnan(want[0]) == bad
         assert bad or _close(got, want, MTOL)[0], (got, want)
         assert int(res.stats["fixed_point_overflow"]) == 0
+
+
+def test_exact_tangents_of_a_fixed_point_sum():
+    """bins of opposite cotangents cancel to ~1e-5 of their size: the exact sums to float64 keep the difference, as the
+    adjoint's exact sum does (rounded to float32 per bin it would be off by ~1e-3)."""
+    n = tm._api.LANES_PAIR_ITEMS
+
+    def item(t, x, th):
+        def body(c):
+            k, t = c
+            w = jnp.exp(jnp.sin(jnp.log(x)))       # (the same in every bin, but for a few items of the last)
+            w = jnp.where((k == 15) & (x > 3.9999), w * 1.5, w)
+            return k + 1, t.add("h", k, th[0] * w)
+        return lax.while_loop(lambda c: c[0] < 16, body, (np.int32(0), t))[1]
+    x = np.linspace(0.25, 4.0, n).astype(np.float32)
+    th = np.array([1.5], np.float32)
+    ct = {"h": np.tile(np.array([1.0, -1.0], np.float32), 8)}
+    g = {}
+    for mode in ("auto", "reverse"):
+        f = tm.vmap(item, outputs={"h": tm.Sum((16,), fixed_point=True)}, in_axes=(0, None), grad_mode=mode)
+        g[mode] = _np(tm.vjp(f, x, th, argnums=1)[1](ct))
+    assert g["auto"][0] != 0.0 and np.allclose(g["auto"], g["reverse"], rtol=1e-6, atol=0.0), g

@@ -114,6 +114,14 @@ def test_vjp_takes_lanes_where_they_cost_less_than_two_launches():
     assert plan(problems.mapped("random_walk"), args, 2, False) is None
     assert plan(problems.mapped("barrier"), problems.PROBLEMS["barrier"]["inputs"](64)[0], 2, True) is None
 
+    # (a fixed-point float32 sum's tangents too are exact to float64; a scaled sum's would be rounded to its scale)
+    for dt in (np.float32, np.float64):
+        f = tm.vmap(rw["item"], outputs={"hist": tm.Sum((64,), dtype=dt, fixed_point=True)}, in_axes=rw["in_axes"])
+        assert (plan(f, args, 2, True) is not None) == (dt == np.float32)
+        if dt == np.float32:
+            q = _api._jvp_prog(f._prepare(args)[0], (False,), (False, True), 3, "exact")
+            assert [(t.dtype, t.exact) for t in q.tallies] == [(dt, True)] + [(np.float64, True)] * 3
+
     def with_result(t, *a):
         t, k = rw["item"](t, *a)
         return t, (k, a[2][0] * 2.0)
