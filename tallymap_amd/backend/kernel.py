@@ -57,6 +57,7 @@ CLAIM_NS = 20_000          # reserve when a chunk lasted less than this many ns
 SHARDS = 64                # item ranges with a claim counter each (one per lane of the wave that looks for items left)
 SHARD0 = 64                # ctl word of the first range's counter (u64), SHARD_WORDS words apart (256 bytes)
 SHARD_WORDS = 64
+IL_CHUNKS = 4              # chunks of a block, where the ranges are blocks dealt out in turn (tape programs)
 RC_WORDS = SHARDS * SHARD_WORDS + 64    # u32 words of a Records output's counters: a u64 of slots claimed per segment of
                            # its raw slots (SHARD_WORDS apart), then (u64) the records appended and the launch's waves
 RC_TOTAL = SHARDS * SHARD_WORDS // 2    # u64 index of the records appended among them
@@ -1279,8 +1280,6 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append(f"  u64* const tm_shc = tm_ctr + {SHARD0 // 2};")
     body.append(f"  const u64 tm_shn = (((u64)n_items + {SHARDS * chunk - 1}u) / {SHARDS * chunk}u) * {chunk}u;")
     body.append(f"  u32 tm_sh = blockIdx.x % {SHARDS}u;")
-    if tape_w:
-        body.append(f"  const u64 tm_nc = ((u64)n_items + {chunk - 1}u) / {chunk}u;                   // chunks")
     body.append("  u64 tm_left = tm_shn;")
     body.append(f"  const u64 tm_shw = (tm_grid * {wpb}u + {SHARDS - 1}u) / {SHARDS}u;")
     body.append("  i32 tm_drop = 0;")
@@ -1316,10 +1315,12 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     # and, once that is used up, from the next range that has items left, found with one load of all counters
     # (a lane each).  A wave learns that no items are left from one such load.  A launch of at most one chunk per
     # wave claims nothing: wave w takes chunk w.
-    # A tape program's ranges deal the chunks out in turn instead (range s: chunks s, s + SHARDS, ...): the rows of its
-    # tape lie in item order, and the resident waves then write and read one window that moves through them, not 64.
-    # The 68.4M-particle shower's tree adjoint, tapes of up to 16 GiB: 29.7 ms with contiguous ranges, 26.1 so
-    # (slab's taped gradient at 500,009 items: 329 us and 328).
+    # A tape program's ranges are blocks of IL_CHUNKS chunks dealt out in turn instead (range s: blocks s, s + SHARDS, ...),
+    # a chunk per claim: the rows of its tape lie in item order, and the resident waves then write and read one window
+    # that moves through them, not 64.  The 68.4M-particle shower's tree adjoint, tapes of up to 16 GiB, 29.7 ms with
+    # contiguous ranges, 26.3 so; the quickstart's item gradients at 4,194,304 items 1,630 us and 667 (blocks of one
+    # chunk 672; slab's replay gradient at 1,048,576 519 with one, 505 with 4 or 16, 524 contiguous; transport's lost, 684
+    # -> 703).
     # A wave that used up its last reservation in less than CLAIM_NS ns reserves RESERVE chunks per claim while its
     # range has more than that many chunks left per wave: a claim is a ~1 us round trip that the whole wave waits
     # for.  The pace is read from the 100 MHz real-time counter at claims only.
@@ -1328,30 +1329,36 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("          if (tm_rv >= tm_re && tm_one) {")
     body.append("            tm_rv = (u64)tm_wid * tm_ch;")
     body.append("            tm_re = tm_rv + tm_ch < (u64)n_items ? tm_rv + tm_ch : (u64)n_items;")
-    body.append("          } else if (tm_rv >= tm_re) {")
-    body.append("            const u64 tm_now = __builtin_amdgcn_s_memrealtime();")
-    body.append(f"            const bool tm_big = tm_t0 != 0ull && (tm_now - tm_t0) * 10ull < tm_rc * {CLAIM_NS}ull "
-                f"&& tm_left > tm_shw * {resv}ull;")
-    body.append(f"            tm_rc = tm_big ? {RESERVE}u : 1u;")
-    body.append("            tm_t0 = tm_now;")
-    body.append("            while (true) {")
     il = tape_w > 0
-    if il:
-        body.append(f"              const u64 tm_sl = tm_range(tm_nc, tm_sh, {SHARDS}u) * {chunk}u;")
+    body.append("          } else if (tm_rv >= tm_re) {")
+    if not il:
+        body.append("            const u64 tm_now = __builtin_amdgcn_s_memrealtime();")
+        body.append(f"            const bool tm_big = tm_t0 != 0ull && (tm_now - tm_t0) * 10ull < tm_rc * {CLAIM_NS}ull "
+                    f"&& tm_left > tm_shw * {resv}ull;")
+        body.append(f"            tm_rc = tm_big ? {RESERVE}u : 1u;")
+        body.append("            tm_t0 = tm_now;")
+    body.append("            while (true) {")
+    if il:                     # (the counter counts the range's chunks; the last block may lack some)
+        body.append(f"              const u64 tm_nc = ((u64)n_items + {chunk - 1}u) / {chunk}u;")
+        body.append(f"              const u64 tm_b = tm_claim(tm_shc + tm_sh * {SHARD_WORDS // 2}u, 1u);")
+        body.append(f"              const u64 tm_k = (tm_b / {IL_CHUNKS}u * {SHARDS}u + tm_sh) * {IL_CHUNKS}u + tm_b % {IL_CHUNKS}u;")
+        body.append("              if (tm_k < tm_nc) {")
+        body.append(f"                tm_rv = tm_k * {chunk}u;")
+        body.append(f"                tm_re = tm_rv + {chunk}u < (u64)n_items ? tm_rv + {chunk}u : (u64)n_items;")
+        body.append("                break;")
+        body.append("              }")
+        body.append(f"              const u64 tm_ll = tm_range((tm_nc + {IL_CHUNKS - 1}u) / {IL_CHUNKS}u, (u32)tm_lane(), "
+                    f"{SHARDS}u) * {IL_CHUNKS}u;")
     else:
         body.append("              const u64 tm_sb = tm_shn * tm_sh < (u64)n_items ? tm_shn * tm_sh : (u64)n_items;")
         body.append("              const u64 tm_sl = tm_sb + tm_shn < (u64)n_items ? tm_shn : (u64)n_items - tm_sb;")
-    base = "" if il else "tm_sb + "
-    body.append(f"              const u64 tm_b = tm_claim(tm_shc + tm_sh * {SHARD_WORDS // 2}u, tm_rc * {chunk}u);")
-    body.append("              if (tm_b < tm_sl) {")
-    body.append(f"                tm_rv = {base}tm_b;")
-    body.append(f"                tm_re = {base}(tm_b + tm_rc * {chunk}u < tm_sl ? tm_b + tm_rc * {chunk}u : tm_sl);")
-    body.append(f"                tm_left = {base}tm_sl - tm_re;")
-    body.append("                break;")
-    body.append("              }")
-    if il:
-        body.append(f"              const u64 tm_ll = tm_range(tm_nc, (u32)tm_lane(), {SHARDS}u) * {chunk}u;")
-    else:
+        body.append(f"              const u64 tm_b = tm_claim(tm_shc + tm_sh * {SHARD_WORDS // 2}u, tm_rc * {chunk}u);")
+        body.append("              if (tm_b < tm_sl) {")
+        body.append("                tm_rv = tm_sb + tm_b;")
+        body.append(f"                tm_re = tm_sb + (tm_b + tm_rc * {chunk}u < tm_sl ? tm_b + tm_rc * {chunk}u : tm_sl);")
+        body.append("                tm_left = tm_sb + tm_sl - tm_re;")
+        body.append("                break;")
+        body.append("              }")
         body.append("              const u64 tm_lb = tm_shn * (u64)tm_lane() < (u64)n_items ? tm_shn * (u64)tm_lane() : (u64)n_items;")
         body.append("              const u64 tm_ll = tm_lb + tm_shn < (u64)n_items ? tm_shn : (u64)n_items - tm_lb;")
     body.append(f"              const u64 tm_lv = __hip_atomic_load(tm_shc + tm_lane() * {SHARD_WORDS // 2}, "
@@ -1363,17 +1370,12 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
     body.append("              tm_rc = 1u;")
     body.append("            }")
     body.append("          }")
-    if il:             # (the reservation counts the range's own items, whole chunks; the last chunk may be short)
-        body.append(f"          const u64 tm_b = tm_one ? tm_rv : tm_rv >= tm_re ? (u64)n_items : "
-                    f"(tm_rv / {chunk}u * {SHARDS}u + tm_sh) * {chunk}u;")
-    else:
-        body.append("          const u64 tm_b = tm_rv;")
+    body.append("          const u64 tm_b = tm_rv;")
     body.append("          if (tm_b >= (u64)n_items) {")
     body.append("            tm_more = false;")
     body.append("          } else {")
-    lim = "(tm_one ? tm_re : (u64)n_items)" if il else "tm_re"
-    body.append(f"            tm_cb = tm_b; tm_cur = 0u; tm_end = (u32)(tm_b + {chunk}u < {lim} ? {chunk}ull : {lim} - tm_b);")
-    body.append(f"            tm_rv += {f'tm_one ? tm_end : {chunk}u' if il else 'tm_end'};")
+    body.append(f"            tm_cb = tm_b; tm_cur = 0u; tm_end = (u32)(tm_b + {chunk}u < tm_re ? {chunk}ull : tm_re - tm_b);")
+    body.append("            tm_rv = tm_b + tm_end;")
     if W:
         body.append(f"            for (u32 q = (u32)tm_lane(); q < {chunk}u; q += 64u) {{")
         body.append("              const u64 t = tm_cb + q;")

@@ -348,8 +348,8 @@ TM_DFN i64 tm_qclaim(u64* ctr, bool when) {
   return when ? (i64)(b + tm_rank(m)) : -1;
 }
 
-// chunks of range s when nc chunks are dealt out to S ranges in turn
-TM_FN u64 tm_range(u64 nc, u32 s, u32 S) { return nc > s ? (nc - s + S - 1u) / S : 0ull; }
+// blocks of range s when n blocks are dealt out to S ranges in turn
+TM_FN u64 tm_range(u64 n, u32 s, u32 S) { return n > s ? (n - s + S - 1u) / S : 0ull; }
 
 // A Records output's slot claim (reference _tally.py:141-160): a wave takes raw slots from a private batch of TM_RB
 // consecutive slots, refilled with one atomic per TM_RB slots.  The batch state (base, slots left, records appended)
