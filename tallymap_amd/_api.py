@@ -601,7 +601,7 @@ def _truncation(trunc, o, N):
     if trunc is not None:
         return trunc, o.n_truncated
     import torch
-    z = torch.zeros((N,), dtype=torch.bool, device="cuda")
+    z = torch.zeros(((N + 3) // 4,), dtype=torch.int32, device="cuda").view(torch.bool)[:N]     # (a word per store)
     # (without a cap the launch counts no truncated children either: its zero, of a buffer of 20 bytes and not of z,
     # which a kept count would keep)
     return z, o.stats[ST["children_truncated"]]
