@@ -57,14 +57,14 @@ def _classes(*counts):
     return {"SQ_INSTS_VALU_" + c: float(n) for c, n in zip(VALU_CLASSES, counts)}
 
 
-MEASURED = {"fused": {"code": "fecd2447bd79fc61", "traffic": 82_477_514, "valu_insts": 6.1971e+09,
-                       "valu_classes": _classes(1.836e+09, 4.837e+07, 1.405e+08, 8.641e+07, 0, 0,
+MEASURED = {"fused": {"code": "26314324dbd20248", "traffic": 82_442_873, "valu_insts": 6.1977e+09,
+                       "valu_classes": _classes(1.836e+09, 4.839e+07, 1.405e+08, 8.642e+07, 0, 0,
                                                 1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
-            "forward": {"code": "a7ef3cc5a67dd356", "traffic": 83_846_204, "valu_insts": 6.1290e+09,
+            "forward": {"code": "208aae0f27d01e41", "traffic": 83_825_685, "valu_insts": 6.1289e+09,
                         "valu_classes": _classes(1.836e+09, 4.838e+07, 1.404e+08, 8.639e+07, 0, 0,
                                                  1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
-            "gradient": {"code": "47f260042cd43e9e", "traffic": 62_372_947, "valu_insts": 5.8874e+09,
-                         "valu_classes": _classes(1.739e+09, 4.388e+07, 1.406e+08, 5.411e+07, 0, 0,
+            "gradient": {"code": "47f260042cd43e9e", "traffic": 62_292_636, "valu_insts": 5.8881e+09,
+                         "valu_classes": _classes(1.739e+09, 4.389e+07, 1.406e+08, 5.412e+07, 0, 0,
                                                   1.675e+08, 1.186e+08, 5.375e+08, 5.173e+06, 1.082e+08)}}
 
 

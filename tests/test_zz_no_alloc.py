@@ -118,3 +118,37 @@ def test_noalloc_allocates_nothing_after_the_first_call():
     assert free1 == free0, (free0, free1)
     for a, b in zip(first, second):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
+@pytest.mark.parametrize("name, flags", [("c1", 2), ("random_walk", 8)])
+def test_noalloc_plain_sums_in_a_graph(name, flags):
+    """plain float32 sums of a spread launch (its float64 sums are in a ctl of the caller's, read by tm_post: of the
+    program's own, or launched for them alone) and of one that does not spread, captured and replayed with eager work
+    between the replays: the eager launch's results."""
+    import torch
+
+    from tallymap_amd import problems
+    cfg = configs.C1 if name == "c1" else dict(problems.PROBLEMS[name], max_steps=None)
+    N = 400_000
+    args = configs.c1_inputs(N) if name == "c1" else cfg["inputs"](N)[0]
+    c = B.compiled(_prog(cfg, args, exact=False), {})
+    L = c.layout
+    assert L.flags == flags and L.spread > 0 and L.r_ctl not in L.scratch
+    for n in (3_000, N):
+        print("case:", name, n, flush=True)
+        ins = _ins([np.asarray(a)[:n] if ax == 0 else a for a, ax in zip(args, cfg["in_axes"])], cfg["in_axes"])
+        ref = B.launch(c, ins, n)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            got = B.launch_noalloc(c, ins, n)
+        for _ in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            for r in L.r_out.values():
+                a, b = got[r - L.n_in].double(), ref[r - L.n_in].double()
+                assert bool((b > 0).any()) and torch.allclose(a, b, rtol=2e-6, atol=0.0), (n, a, b)
+            for r in L.r_ys:
+                assert torch.equal(got[r - L.n_in], ref[r - L.n_in]), n
+            B.launch(c, ins, n)
+            torch.cuda.synchronize()
