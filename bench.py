@@ -57,13 +57,13 @@ def _classes(*counts):
     return {"SQ_INSTS_VALU_" + c: float(n) for c, n in zip(VALU_CLASSES, counts)}
 
 
-MEASURED = {"fused": {"code": "26314324dbd20248", "traffic": 82_442_873, "valu_insts": 6.1977e+09,
-                       "valu_classes": _classes(1.836e+09, 4.839e+07, 1.405e+08, 8.642e+07, 0, 0,
-                                                1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
-            "forward": {"code": "208aae0f27d01e41", "traffic": 83_825_685, "valu_insts": 6.1289e+09,
+MEASURED = {"fused": {"code": "5e98387efe596d3b", "traffic": 82_543_940, "valu_insts": 6.1959e+09,
+                       "valu_classes": _classes(1.835e+09, 4.835e+07, 1.404e+08, 8.638e+07, 0, 0,
+                                                1.673e+08, 1.184e+08, 5.370e+08, 5.173e+06, 1.405e+08)},
+            "forward": {"code": "1cdc3db81d2bc00d", "traffic": 83_894_085, "valu_insts": 6.1294e+09,
                         "valu_classes": _classes(1.836e+09, 4.838e+07, 1.404e+08, 8.639e+07, 0, 0,
                                                  1.674e+08, 1.185e+08, 5.371e+08, 5.173e+06, 1.405e+08)},
-            "gradient": {"code": "47f260042cd43e9e", "traffic": 62_292_636, "valu_insts": 5.8881e+09,
+            "gradient": {"code": "47f260042cd43e9e", "traffic": 62_469_443, "valu_insts": 5.8878e+09,
                          "valu_classes": _classes(1.739e+09, 4.389e+07, 1.406e+08, 5.412e+07, 0, 0,
                                                   1.675e+08, 1.186e+08, 5.375e+08, 5.173e+06, 1.082e+08)}}
 

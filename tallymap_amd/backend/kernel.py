@@ -1235,6 +1235,9 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
             body.append(f"  __shared__ {ct} tm_sh{k}[{n}];")
             body.append(f"  for (int i = threadIdx.x; i < {n}; i += TM_BLOCK) tm_sh{k}[i] = ({ct})0;")
     body.append("//TM_COUNT_DECLS")
+    if wide:                   # (a spread launch: more workgroups than its items fill; read by the flush)
+        body.append("  __shared__ u32 tm_spread_s;")
+        body.append("  if (threadIdx.x == 0) tm_spread_s = (u64)tm_grid * TM_BLOCK >= (u64)n_items + TM_BLOCK ? 1u : 0u;")
     for i in staged:
         a = bav[i]
         ct = ctype(a.dtype)
@@ -1563,8 +1566,8 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
         src.append(f"#define TM_CN{k}(e) ({copy_of('(e)', ccopy[k])})")
     if priv:
         body.append("  __syncthreads();")
-        if wide:               # (a spread launch: more workgroups than its items fill)
-            body.append(f"  const bool tm_wide = (u64)tm_grid * TM_BLOCK >= (u64)n_items + TM_BLOCK;")
+        if wide:
+            body.append("  const bool tm_wide = __builtin_amdgcn_readfirstlane(tm_spread_s) != 0u;")
         for k in priv:
             s = prog.tallies[k]
             if s.exact:
@@ -1591,7 +1594,7 @@ def build(prog, block=BLOCK, schedule="step", refill=1, chunk=CHUNK, compact=COM
                 body.append(f"  for (int i = threadIdx.x; i < {s.S}; i += TM_BLOCK) {{ const {ct} x = tm_sh{k}[i]; "
                             f"if (x != 0) tm_gadd_u64(&((u64*)P.p[{r_out[k]}])[i], (u64)x); }}")
             elif s.dtype == C.F32:
-                gw = f"(double*)tm_ctr + {wide[k]} + i" if k in wide else None
+                gw = f"(double*)P.p[{r_ctl}] + {wide[k]} + i" if k in wide else None
                 go = f"&((float*)P.p[{r_out[k]}])[i]"
 
                 def flush(total, cond, x32, x64):
