@@ -1,6 +1,6 @@
 """Forward parity on the GPU: the HIP path (tm.vmap -> libtallymap_rocm.so tm_launch -> gfx950 kernel) against the
 oracle on the same seeded inputs.  Integer per-item results and stats bit-exact; f32 tallies within 1e-5 relative of
-the oracle's float64 re-summation (BASELINE north_star)."""
+the oracle's float64 re-summation."""
 import numpy as np
 import pytest
 

@@ -1,5 +1,5 @@
 """Reverse mode on the GPU: the replay adjoint kernel against the oracle's forward-mode (dual number) gradients.
-Gradients within 1e-4 relative (BASELINE north_star); the per-item cotangents bitwise independent of the replay's
+Gradients within 1e-4 relative; the per-item cotangents bitwise independent of the replay's
 schedule, tape size and checkpoint count (reference tests/reverse.py:216); truncation makes every cotangent NaN (reference _primitive.py:586-594)."""
 import numpy as np
 import pytest
